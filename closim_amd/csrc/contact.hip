@@ -1598,6 +1598,313 @@ __global__ void __launch_bounds__(kKillBlock) k_kill_run(const KillRec* __restri
   if (threadIdx.x == 0) *rounds_out = round;
 }
 
+// ---- the sweep as a dataflow in one work-group ------------------------------
+// k_kill_run's round costs an L2 round trip (the released contact's record),
+// and the critical path of a stack of sheets is 16,000 contacts of 139,000.
+// Here every contact knows its rank on each of its vertices, and a vertex in
+// LDS carries its velocity and the number of its contacts that have run: a
+// contact may run when each of its vertices has run exactly `rank` contacts.
+// The contacts are dealt to the 64 lanes of wave 0 by their first cloth
+// vertex (id % 64: neighbours, which wait for each other, on different lanes;
+// by a random slot the two sheets below take 92,000 passes instead of 21,000),
+// each lane's in list order, so the first unfinished
+// contact of the whole list is always at the head of its lane and ready: one
+// pass of the wave reads every head's vertices (velocity and count in two
+// 16-byte LDS reads each), runs the ready ones and writes them back.  Ready
+// heads share no vertex.  A pass is bound by LDS latency and the FP64 chain of
+// one contact; waves 1..4 keep each lane's next records in an LDS ring (wave w
+// the w-th 16 bytes of a record), so no pass waits for memory.
+// Measured (kernel): two 33x33 sheets, 139,462 contacts, depth 15,802: 79.9 ms
+// with k_kill_run<false>, 16.2 ms here; the 256x256 drape on its sphere, 5,164
+// contacts, depth 1,702: 2.35 ms with the LDS form of k_kill_run, 1.35 ms here.
+
+constexpr uint32_t kFlowLanes = 64, kFlowRing = 8, kFlowBatch = 4;
+constexpr int kFlowWaves = 5;                    // the consumer and four producers
+constexpr uint32_t kFlowMaxRank = (1u << 18) - 1;
+constexpr uint32_t kFlowMaxSlot = (1u << 12) - 1;
+
+// 64 bytes: four 16-byte chunks.  meta[s]: LDS slot of vertex s (bits 0-11),
+// bit 12 set when there is none (static, or a floor contact's unused slots),
+// the rank (bits 14-31); meta[0] bit 13 and meta[1] bit 13: the kind's bits.
+struct alignas(16) KillFlowRec {
+  double nx, ny, nz, w0, w1, w2;
+  uint32_t meta[4];
+};
+static_assert(sizeof(KillFlowRec) == 64, "four chunks");
+
+// One vertex: velocity, contacts run, length of the longest chain of contacts
+// ending here.
+struct FlowVert {
+  double x, y, z;
+  uint32_t done, level;
+};
+
+// kill_contact on velocities held in registers, the same operations in the
+// same order.  kFull: all four vertices exist; otherwise on[s] says which (a
+// missing vertex adds nothing to a triangle's sum and stands for a zero
+// velocity in an edge pair; its register is not written back).  The sums start
+// from their first term: starting from zero could only change the sign of a
+// zero, which no comparison below sees.
+template <bool kFull>
+__device__ __forceinline__ void flow_vt(const KillFlowRec& c, const bool* on, FlowVert* q) {
+  double tx = 0, ty = 0, tz = 0;
+  const double ws[3] = {c.w0, c.w1, c.w2};
+  if constexpr (kFull) {
+    tx = ws[0] * q[1].x + ws[1] * q[2].x + ws[2] * q[3].x;
+    ty = ws[0] * q[1].y + ws[1] * q[2].y + ws[2] * q[3].y;
+    tz = ws[0] * q[1].z + ws[1] * q[2].z + ws[2] * q[3].z;
+  } else {
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      tx = on[k + 1] ? tx + ws[k] * q[k + 1].x : tx;
+      ty = on[k + 1] ? ty + ws[k] * q[k + 1].y : ty;
+      tz = on[k + 1] ? tz + ws[k] * q[k + 1].z : tz;
+    }
+  }
+  const double rel = (q[0].x - tx) * c.nx + (q[0].y - ty) * c.ny + (q[0].z - tz) * c.nz;
+  if (rel < 0) {
+    const double j = -0.5 * rel;
+    q[0].x += j * c.nx;
+    q[0].y += j * c.ny;
+    q[0].z += j * c.nz;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const double jw = j * ws[k];
+      q[k + 1].x -= jw * c.nx;
+      q[k + 1].y -= jw * c.ny;
+      q[k + 1].z -= jw * c.nz;
+    }
+  }
+}
+
+template <bool kFull>
+__device__ __forceinline__ void flow_ee(const KillFlowRec& c, const bool* on, FlowVert* q) {
+  double P[4][3];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    P[k][0] = kFull || on[k] ? q[k].x : 0.0;
+    P[k][1] = kFull || on[k] ? q[k].y : 0.0;
+    P[k][2] = kFull || on[k] ? q[k].z : 0.0;
+  }
+  double d[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) d[k] = (P[0][k] + P[1][k]) / 2 - (P[2][k] + P[3][k]) / 2;
+  const double rel = d[0] * c.nx + d[1] * c.ny + d[2] * c.nz;
+  if (rel < 0) {
+    const double j = -0.25 * rel;
+    const double jx = j * c.nx, jy = j * c.ny, jz = j * c.nz;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      q[k].x += jx;
+      q[k].y += jy;
+      q[k].z += jz;
+      q[k + 2].x -= jx;
+      q[k + 2].y -= jy;
+      q[k + 2].z -= jz;
+    }
+  }
+}
+
+__device__ __forceinline__ void frozen_verts(const Frozen& c, int32_t* vs) {
+  vs[0] = c.kind == 1 ? c.a : c.p;
+  vs[1] = c.kind == 2 ? -1 : c.kind == 0 ? c.a : c.b;
+  vs[2] = c.kind == 2 ? -1 : c.kind == 0 ? c.b : c.c;
+  vs[3] = c.kind == 2 ? -1 : c.kind == 0 ? c.c : c.d;
+}
+
+// the lane of every contact (sort key) and its list position
+__global__ void k_flow_owner(const Frozen* __restrict__ act, uint32_t C, uint64_t* key, uint32_t* idx) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= C) return;
+  int32_t vs[4];
+  frozen_verts(act[i], vs);
+  uint32_t lane = i % kFlowLanes;  // no cloth vertex (never emitted): any lane
+  for (int s = 3; s >= 0; s--)
+    if (vs[s] >= 0) lane = (uint32_t)vs[s] % kFlowLanes;
+  key[i] = lane;
+  idx[i] = i;
+}
+
+// record k of the lane order; pos[i]: where contact i went
+__global__ void k_flow_rec(const Frozen* __restrict__ act, uint32_t C, const uint32_t* __restrict__ vslot,
+                           const uint32_t* __restrict__ idx, KillFlowRec* rec, uint32_t* pos) {
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= C) return;
+  const uint32_t i = idx[k];
+  const Frozen c = act[i];
+  int32_t vs[4];
+  frozen_verts(c, vs);
+  KillFlowRec r;
+  r.nx = c.nx; r.ny = c.ny; r.nz = c.nz;
+  r.w0 = c.w0; r.w1 = c.w1; r.w2 = c.w2;
+  for (int s = 0; s < 4; s++) r.meta[s] = vs[s] >= 0 ? vslot[vs[s]] : 1u << 12;
+  r.meta[0] |= ((uint32_t)c.kind & 1u) << 13;
+  r.meta[1] |= ((uint32_t)c.kind >> 1) << 13;
+  rec[k] = r;
+  pos[i] = k;
+}
+
+// per incidence entry: the contact's rank on the vertex (each meta word is
+// written by one entry)
+__global__ void k_flow_rank(const uint32_t* __restrict__ v_off, const uint32_t* __restrict__ v_ent,
+                            const uint32_t* __restrict__ ent_vtx, uint32_t E, const uint32_t* __restrict__ pos,
+                            KillFlowRec* rec) {
+  const uint32_t h = blockIdx.x * blockDim.x + threadIdx.x;
+  if (h >= E) return;
+  const uint32_t e = v_ent[h];
+  rec[pos[e >> 3]].meta[e & 7] |= (h - v_off[ent_vtx[h]]) << 14;
+}
+
+struct alignas(16) FlowZ {
+  double z;
+  uint32_t done, level;
+};
+
+// first k with key[k] >= lane
+__device__ __forceinline__ uint32_t flow_lower(const uint64_t* __restrict__ key, uint32_t C, uint32_t lane) {
+  uint32_t lo = 0, hi = C;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) / 2;
+    if (key[mid] < lane) lo = mid + 1;
+    else hi = mid;
+  }
+  return lo;
+}
+
+__global__ void __launch_bounds__(kFlowWaves * kWave) k_kill_flow(const KillFlowRec* __restrict__ rec,
+                                                                  const uint64_t* __restrict__ key, uint32_t C,
+                                                                  const uint32_t* __restrict__ cverts, uint32_t nv,
+                                                                  double* v, uint32_t* rounds_out) {
+  extern __shared__ __align__(16) unsigned char flow_lds[];
+  double2* Vxy = reinterpret_cast<double2*>(flow_lds);         // [nv] x, y
+  FlowZ* Vz = reinterpret_cast<FlowZ*>(Vxy + nv);              // [nv] z, done, level
+  uint4* ring = reinterpret_cast<uint4*>(Vz + nv);             // [kFlowRing][4][kFlowLanes]
+  uint32_t* tails = reinterpret_cast<uint32_t*>(ring + kFlowRing * 4 * kFlowLanes);  // [kFlowLanes][4]: records in the ring
+  uint32_t* heads = tails + 4 * kFlowLanes;                    // [kFlowLanes]: records taken out
+  const uint32_t lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
+  for (uint32_t k = threadIdx.x; k < nv; k += blockDim.x) {
+    const size_t u = cverts[k];
+    Vxy[k] = make_double2(v[u * 3], v[u * 3 + 1]);
+    Vz[k] = FlowZ{v[u * 3 + 2], 0, 0};
+  }
+  for (uint32_t k = threadIdx.x; k < 5 * kFlowLanes; k += blockDim.x) tails[k] = 0;  // heads follow
+  const uint32_t beg = flow_lower(key, C, lane), cnt = flow_lower(key, C, lane + 1) - beg;
+  __syncthreads();
+  if (wid) {
+    // producers: each pass moves up to kFlowBatch records of every lane, and
+    // the loop ends when all records of the wave's lanes are in the ring
+    // (the consumer never stops taking them out)
+    const uint4* src = reinterpret_cast<const uint4*>(rec) + (wid - 1);
+    uint32_t tail = 0;
+    while (__ballot(tail < cnt)) {
+      const uint32_t head = __hip_atomic_load(&heads[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      const uint32_t nb = min(min(cnt - tail, head + kFlowRing - tail), kFlowBatch);
+      if (!__ballot(nb != 0)) {
+        __builtin_amdgcn_s_sleep(1);
+        continue;
+      }
+      // unconditional loads (past the lane's last record: some record of the
+      // list), so that all are in flight together
+      uint4 q[kFlowBatch];
+#pragma unroll
+      for (uint32_t b = 0; b < kFlowBatch; b++) q[b] = src[(size_t)min(beg + tail + b, C - 1) * 4];
+#pragma unroll
+      for (uint32_t b = 0; b < kFlowBatch; b++)
+        if (b < nb) ring[((tail + b) % kFlowRing * 4 + wid - 1) * kFlowLanes + lane] = q[b];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+      tail += nb;
+      if (nb) __hip_atomic_store(&tails[lane * 4 + wid - 1], tail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+  } else {
+    // `c` is the lane's head; `nxt` the record after it, read from the ring
+    // while the head waits or runs
+    uint32_t taken = 0, avail = 0, top = 0;  // records taken from the ring, known to be in it, longest chain
+    bool have = false, have_nxt = false;
+    KillFlowRec c = {}, nxt = {};
+    while (__ballot(have || have_nxt || taken < cnt)) {
+      FlowVert q[4];
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const uint32_t k = c.meta[s] & kFlowMaxSlot;
+        const FlowZ zd = Vz[k];
+        const double2 xy = Vxy[k];
+        q[s] = FlowVert{xy.x, xy.y, zd.z, zd.done, zd.level};
+      }
+      if (!have_nxt && taken < cnt) {
+        if (taken == avail) {
+          uint32_t t[4];
+#pragma unroll
+          for (int k = 0; k < 4; k++)
+            t[k] = __hip_atomic_load(&tails[lane * 4 + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          avail = min(min(t[0], t[1]), min(t[2], t[3]));
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        }
+        if (taken < avail) {
+          uint4* dst = reinterpret_cast<uint4*>(&nxt);
+#pragma unroll
+          for (int k = 0; k < 4; k++) dst[k] = ring[(taken % kFlowRing * 4 + k) * kFlowLanes + lane];
+          taken++;
+          have_nxt = true;
+        }
+      }
+      bool on[4], ready = have;
+      uint32_t level = 0;
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        on[s] = !(c.meta[s] & (1u << 12));
+        ready = ready & (!on[s] | (q[s].done == c.meta[s] >> 14));
+        level = max(level, on[s] ? q[s].level : 0u);
+      }
+      // most passes run contacts of one kind with four cloth vertices
+      const bool full = on[0] & on[1] & on[2] & on[3];
+      const bool odd = __ballot(ready && !full) != 0;
+      if (ready) {
+        const bool ee = (c.meta[0] >> 13) & 1u, floor = (c.meta[1] >> 13) & 1u;
+        if (ee) {
+          if (odd) flow_ee<false>(c, on, q);
+          else flow_ee<true>(c, on, q);
+        } else if (!floor) {
+          if (odd) flow_vt<false>(c, on, q);
+          else flow_vt<true>(c, on, q);
+        } else if (q[0].y < 0) {
+          q[0].y = 0;
+        }
+        level++;
+        top = max(top, level);
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+          if (!odd || on[s]) {
+            const uint32_t k = c.meta[s] & kFlowMaxSlot;
+            Vxy[k] = make_double2(q[s].x, q[s].y);
+            Vz[k] = FlowZ{q[s].z, q[s].done + 1, level};
+          }
+        have = false;
+      }
+      if (!have && have_nxt) {
+        c = nxt;
+        have = true;
+        have_nxt = false;
+        // the record is out of the ring: its place may be filled again
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __hip_atomic_store(&heads[lane], taken, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+    }
+    for (int off = kWave / 2; off > 0; off >>= 1) top = max(top, (uint32_t)__shfl_down((int)top, off, kWave));
+    if (lane == 0) *rounds_out = top;
+  }
+  __syncthreads();
+  for (uint32_t k = threadIdx.x; k < nv; k += blockDim.x) {
+    const size_t u = cverts[k];
+    v[u * 3] = Vxy[k].x;
+    v[u * 3 + 1] = Vxy[k].y;
+    v[u * 3 + 2] = Vz[k].z;
+  }
+}
+
+static size_t flow_lds_bytes(uint32_t nv) {
+  return (size_t)nv * (sizeof(double2) + sizeof(FlowZ)) + (size_t)kFlowRing * 4 * kFlowLanes * sizeof(uint4) + 5 * kFlowLanes * 4;
+}
+
 // checkTrial prims (contact-assembly.ts:497-535) per pair; pairs [0, np)
 // are cloth/cloth, then nsp cloth/static.  Per prim: exact distance at the
 // trial, the swept-box prefilter, then the head of the reference's CCD; the
@@ -1729,17 +2036,16 @@ static int bits_for(uint64_t v) {
   return b;
 }
 
-// Dynamic LDS available to the LDS velocity-filter sweep: the device's
-// opt-in per-work-group maximum (raised for that kernel), less its static LDS.
-static size_t kill_lds_limit() {
+// Dynamic LDS available to a velocity-filter sweep: the device's opt-in
+// per-work-group maximum (raised for that kernel), less its static LDS.
+static size_t dynamic_lds_limit(const void* kernel) {
   int dev = 0, optin = 0, base = 0;
   CS_HIP(hipGetDevice(&dev));
   if (hipDeviceGetAttribute(&optin, hipDeviceAttributeSharedMemPerBlockOptin, dev) != hipSuccess) optin = 0;
   CS_HIP(hipDeviceGetAttribute(&base, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
   size_t lim = (size_t)std::max(optin, base);
   if (lim > (size_t)base &&
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&k_kill_run<true>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)(lim - 64)) != hipSuccess)
+      hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(lim - 64)) != hipSuccess)
     lim = (size_t)base;
   return lim > 64 ? lim - 64 : 0;
 }
@@ -1847,8 +2153,10 @@ struct ContactImpl {
   // per-contact evaluation
   DevBuf<uint8_t> inr;
   DevBuf<KillRec> krec;           // velocity-filter sweep records
+  DevBuf<KillFlowRec> kflow;      // the dataflow sweep's, in lane order
   DevBuf<uint32_t> kcnt, klist;    // counters / frontier lists of the global-memory sweep
   size_t kill_lds_max = 0;         // dynamic LDS the LDS sweep may use
+  size_t flow_lds_max = 0;         // and the dataflow sweep
   DevBuf<double> cg, fr, coeff, dd, hvsum, hterm;
   DevBuf<uint32_t> heads, cverts;
   // lagged friction table
@@ -1986,7 +2294,8 @@ struct ContactImpl {
     v_off.alloc(n + 1);
     heads.alloc(n);
     klist.alloc((size_t)2 * std::max<uint32_t>(n, 1));
-    kill_lds_max = kill_lds_limit();
+    kill_lds_max = dynamic_lds_limit(reinterpret_cast<const void*>(&k_kill_run<true>));
+    flow_lds_max = dynamic_lds_limit(reinterpret_cast<const void*>(&k_kill_flow));
     cverts.alloc(std::max<uint32_t>(n, 1));
     hvsum.alloc((size_t)std::max<uint32_t>(n, 1) * 3);
     hvsum.zero(st);
@@ -2434,6 +2743,22 @@ struct ContactImpl {
     if (!C) return;
     // heads[] (n entries) serves as the vertex -> LDS slot map here
     hipLaunchKernelGGL(k_kill_slots, dim3(grid_for(nv)), dim3(kBlock), 0, st, cverts.ptr, nv, heads.ptr);
+    if (nv <= kFlowMaxSlot && C <= kFlowMaxRank && flow_lds_bytes(nv) <= flow_lds_max) {
+      ensure_sort(C);
+      hipLaunchKernelGGL(k_flow_owner, dim3(grid_for(C)), dim3(kBlock), 0, st, act.ptr, C, akeys.ptr, avals.ptr);
+      const bool in_tmp = radix_sort_pairs(st, akeys.ptr, avals.ptr, akeys_t.ptr, avals_t.ptr, C, 0, 8, sort);
+      kflow.alloc(act_cap);
+      hipLaunchKernelGGL(k_flow_rec, dim3(grid_for(C)), dim3(kBlock), 0, st, act.ptr, C, heads.ptr,
+                         in_tmp ? avals_t.ptr : avals.ptr, kflow.ptr, kcnt.ptr);
+      hipLaunchKernelGGL(k_flow_rank, dim3(grid_for(E)), dim3(kBlock), 0, st, v_off.ptr, v_ent.ptr, ent_vtx.ptr, E,
+                         kcnt.ptr, kflow.ptr);
+      hipLaunchKernelGGL(k_kill_flow, dim3(1), dim3(kFlowWaves * kWave), flow_lds_bytes(nv), st, kflow.ptr,
+                         in_tmp ? akeys_t.ptr : akeys.ptr, C, cverts.ptr, nv, v, &cs.ptr->kill_rounds);
+      CS_LAUNCH_CHECK();
+      sync_cs();
+      diag.filter_rounds = hcs->kill_rounds;
+      return;
+    }
     hipLaunchKernelGGL(k_kill_rec, dim3(grid_for(C)), dim3(kBlock), 0, st, act.ptr, C, heads.ptr, krec.ptr);
     hipLaunchKernelGGL(k_kill_links, dim3(grid_for(E)), dim3(kBlock), 0, st, v_off.ptr, v_ent.ptr, ent_vtx.ptr, E,
                        krec.ptr);

@@ -194,7 +194,8 @@ typedef struct cs_contact_diag {
   double friction_work;
   uint64_t rejected_line_search_steps;
   uint64_t ccd_failures;
-  uint64_t filter_rounds;  /* rounds of the parallel restitution-0 velocity filter (not in the reference) */
+  uint64_t filter_rounds;  /* the restitution-0 velocity filter (not in the reference): the longest chain of contacts
+                              that wait for each other, or the rounds of the round-based sweep */
 } cs_contact_diag;
 
 /* StepStats (src/solver/newton.ts:10-18) plus a few counters the reference
