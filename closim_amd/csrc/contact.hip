@@ -22,6 +22,7 @@
 #include "collide.h"
 #include "contact.h"
 #include "sort.h"
+#include "vsum.h"
 
 namespace cloth {
 
@@ -1109,13 +1110,11 @@ __global__ void __launch_bounds__(kBlock) k_contact_eval(DGeom G, const double* 
 // then friction term) in parallel, then one thread per contact vertex and
 // component adds them in list order.  Components an entry does not touch
 // carry +0, which leaves a sum that started at +0 unchanged.
-__global__ void __launch_bounds__(kBlock) k_grad_terms(uint32_t E, const Frozen* __restrict__ act,
-                                                       const uint32_t* __restrict__ v_ent, CEval ev,
-                                                       double* __restrict__ gterm) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= E) return;
-  double ta[3] = {0, 0, 0}, tb[3] = {0, 0, 0};
-  const uint32_t ent = v_ent[k];
+// t = the entry's distance-gradient term, then its friction term
+__device__ __forceinline__ void grad_term(const Frozen* __restrict__ act, uint32_t ent, const CEval& ev, double* t) {
+  double* ta = t;
+  double* tb = t + 3;
+  for (int q = 0; q < 6; q++) t[q] = 0;
   const uint32_t ci = ent >> 3;
   const int slot = ent & 7;
   if (ev.inr[ci]) {
@@ -1142,11 +1141,30 @@ __global__ void __launch_bounds__(kBlock) k_grad_terms(uint32_t E, const Frozen*
       for (int q = 0; q < 3; q++) tb[q] = fp[q] * ww;
     }
   }
-  for (int q = 0; q < 3; q++) {
-    gterm[(size_t)k * 6 + q] = ta[q];
-    gterm[(size_t)k * 6 + 3 + q] = tb[q];
-  }
 }
+
+__global__ void __launch_bounds__(kBlock) k_grad_terms(uint32_t E, const Frozen* __restrict__ act,
+                                                       const uint32_t* __restrict__ v_ent, CEval ev,
+                                                       double* __restrict__ gterm) {
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= E) return;
+  double t[6];
+  grad_term(act, v_ent[k], ev, t);
+  for (int q = 0; q < 6; q++) gterm[(size_t)k * 6 + q] = t[q];
+}
+
+// the same sums by k_vertex_sums
+struct GradSums {
+  static constexpr bool kPair = true;
+  const Frozen* act;
+  const uint32_t* v_ent;
+  CEval ev;
+  double* ceg;
+  __device__ bool skip() const { return false; }
+  __device__ double init(uint32_t, int) const { return 0.0; }
+  __device__ void term(uint32_t k, double* t) const { grad_term(act, v_ent[k], ev, t); }
+  __device__ void store(uint32_t v, int q, double s) const { ceg[(size_t)v * 3 + q] = s; }
+};
 
 __global__ void __launch_bounds__(kBlock) k_grad_vsum(uint32_t nv, const uint32_t* __restrict__ cverts,
                                                       const uint32_t* __restrict__ v_off,
@@ -1251,13 +1269,8 @@ __global__ void __launch_bounds__(kBlock) k_fric_adj_vsum(uint32_t nv, const uin
 // addDiagEstimate (contact-assembly.ts:436-471): accumulate into diag, the
 // same two passes (a floor contact touches only the y component; +0 added to
 // a positive diagonal leaves it unchanged).
-__global__ void __launch_bounds__(kBlock) k_diag_terms(uint32_t E, const Frozen* __restrict__ act,
-                                                       const uint32_t* __restrict__ v_ent, CEval ev,
-                                                       double* __restrict__ dterm) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= E) return;
-  double t[3] = {0, 0, 0};
-  const uint32_t ent = v_ent[k];
+__device__ __forceinline__ void diag_term(const Frozen* __restrict__ act, uint32_t ent, const CEval& ev, double* t) {
+  t[0] = t[1] = t[2] = 0;
   const uint32_t ci = ent >> 3;
   const int slot = ent & 7;
   if (ev.inr[ci]) {
@@ -1276,8 +1289,29 @@ __global__ void __launch_bounds__(kBlock) k_diag_terms(uint32_t E, const Frozen*
       }
     }
   }
+}
+
+__global__ void __launch_bounds__(kBlock) k_diag_terms(uint32_t E, const Frozen* __restrict__ act,
+                                                       const uint32_t* __restrict__ v_ent, CEval ev,
+                                                       double* __restrict__ dterm) {
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= E) return;
+  double t[3];
+  diag_term(act, v_ent[k], ev, t);
   for (int q = 0; q < 3; q++) dterm[(size_t)k * 3 + q] = t[q];
 }
+
+struct DiagSums {
+  static constexpr bool kPair = false;
+  const Frozen* act;
+  const uint32_t* v_ent;
+  CEval ev;
+  double* diag;
+  __device__ bool skip() const { return false; }
+  __device__ double init(uint32_t v, int q) const { return diag[(size_t)v * 3 + q]; }
+  __device__ void term(uint32_t k, double* t) const { diag_term(act, v_ent[k], ev, t); }
+  __device__ void store(uint32_t v, int q, double s) const { diag[(size_t)v * 3 + q] = s; }
+};
 
 __global__ void __launch_bounds__(kBlock) k_diag_vsum(uint32_t nv, const uint32_t* __restrict__ cverts,
                                                       const uint32_t* __restrict__ v_off,
@@ -2623,7 +2657,9 @@ struct ContactImpl {
       }
     }
     CS_HIP(hipMemsetAsync(ceg, 0, (size_t)n * 3 * sizeof(double), st));
-    if (E) {
+    if (E && use_vertex_groups(E, nv)) {
+      launch_vertex_sums(st, GradSums{act.ptr, v_ent.ptr, cev(), ceg}, nv, cverts.ptr, v_off.ptr);
+    } else if (E) {
       hipLaunchKernelGGL(k_grad_terms, dim3(grid_for(E)), dim3(kBlock), 0, st, E, act.ptr, v_ent.ptr, cev(),
                          hterm.ptr);
       hipLaunchKernelGGL(k_grad_vsum, dim3(grid_for((size_t)nv * 3)), dim3(kBlock), 0, st, nv, cverts.ptr, v_off.ptr,
@@ -2671,7 +2707,9 @@ struct ContactImpl {
 
   void add_diag_estimate(double* dg) {
     if (!C) return;
-    if (E) {
+    if (E && use_vertex_groups(E, nv)) {
+      launch_vertex_sums(st, DiagSums{act.ptr, v_ent.ptr, cev(), dg}, nv, cverts.ptr, v_off.ptr);
+    } else if (E) {
       hipLaunchKernelGGL(k_diag_terms, dim3(grid_for(E)), dim3(kBlock), 0, st, E, act.ptr, v_ent.ptr, cev(),
                          hterm.ptr);
       hipLaunchKernelGGL(k_diag_vsum, dim3(grid_for((size_t)nv * 3)), dim3(kBlock), 0, st, nv, cverts.ptr, v_off.ptr,
@@ -3099,6 +3137,7 @@ DContactHvp ContactSystem::hvp_hook() {
   h.nv = im_->nv;
   h.ent_vtx = im_->ent_vtx.ptr;
   h.term = im_->hterm.ptr;
+  h.dd = im_->dd.ptr;
   h.cverts = im_->cverts.ptr;
   h.vsum = im_->hvsum.ptr;
   h.act = im_->act.ptr;

@@ -27,6 +27,7 @@ struct DContactHvp {
   const uint32_t* ent_vtx = nullptr; // [E] vertex of each entry
   const uint32_t* cverts = nullptr;  // [nv] the vertices with entries
   double* term = nullptr;            // [3E] per-entry terms of the current p
+  double* dd = nullptr;              // [C] dd_c of the current p
   double* vsum = nullptr;            // [3n] contact HVP per vertex (0 off cverts)
 };
 

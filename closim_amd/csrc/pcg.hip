@@ -15,6 +15,7 @@
 #include "elements.h"
 #include "pcg.h"
 #include "schwarz.h"
+#include "vsum.h"
 
 namespace cloth {
 
@@ -88,12 +89,11 @@ __device__ __forceinline__ void hvp_corner(const PcgArgs& a, uint4 cr, const dou
   }
 }
 
-// One contact incidence entry's term at the vertex (applyHvp's addDistGrad).
-__device__ __forceinline__ bool contact_term(const DContactHvp& H, uint32_t ent, const double* __restrict__ p,
-                                             double* c) {
+// One contact incidence entry's term at the vertex (applyHvp's addDistGrad),
+// g = the contact's dd_c.
+__device__ __forceinline__ bool contact_term(const DContactHvp& H, uint32_t ent, double g, double* c) {
   const uint32_t ci = ent >> 3;
   const int slot = ent & 7;
-  const double g = contact_dd(H, ci, p);
   if (g == 0) return false;
   const Frozen& f = H.act[ci];
   if (f.kind == 2) {
@@ -171,7 +171,8 @@ __global__ void __launch_bounds__(kBlock) k_contact_terms(DContactHvp H, const d
   const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= H.E) return;
   double t[3] = {0, 0, 0};
-  if (!contact_term(H, H.v_ent[e], p, t)) t[0] = t[1] = t[2] = 0;
+  const uint32_t ent = H.v_ent[e];
+  if (!contact_term(H, ent, contact_dd(H, ent >> 3, p), t)) t[0] = t[1] = t[2] = 0;
   H.term[(size_t)e * 3] = t[0];
   H.term[(size_t)e * 3 + 1] = t[1];
   H.term[(size_t)e * 3 + 2] = t[2];
@@ -185,6 +186,28 @@ __global__ void __launch_bounds__(kBlock) k_contact_vsum(DContactHvp H, const in
   const int q = t % 3;
   H.vsum[(size_t)v * 3 + q] = ordered_sum<3, 0>(H.term + q, H.v_off[v], H.v_off[v + 1], 0.0);
 }
+
+// The same where vertices have many entries (use_vertex_groups): dd_c once
+// per contact, then k_vertex_sums.
+__global__ void __launch_bounds__(kBlock) k_contact_dd(DContactHvp H, const double* __restrict__ p,
+                                                       const int32_t* done) {
+  if (block_latched(done)) return;
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < H.C) H.dd[i] = contact_dd(H, i, p);
+}
+
+struct HvpSums {
+  static constexpr bool kPair = false;
+  DContactHvp H;
+  const int32_t* done;
+  __device__ bool skip() const { return block_latched(done); }
+  __device__ double init(uint32_t, int) const { return 0.0; }
+  __device__ void term(uint32_t e, double* t) const {
+    const uint32_t ent = H.v_ent[e];
+    if (!contact_term(H, ent, H.dd[ent >> 3], t)) t[0] = t[1] = t[2] = 0;
+  }
+  __device__ void store(uint32_t v, int q, double s) const { H.vsum[(size_t)v * 3 + q] = s; }
+};
 
 // z = M^-1 r at vertex v (Jacobi with the diag > 1e-12 guard, or 3x3 block).
 __device__ __forceinline__ void precond_vertex(const PcgArgs& a, uint32_t v, const double* r3, double* z3) {
@@ -463,7 +486,10 @@ void pcg_iteration(hipStream_t st, const PcgArgs& a, int k) {
 
 // The HVP grid differs from the vector grid; its partial count is passed on.
 void pcg_iteration_hvp(hipStream_t st, const PcgArgs& a, int k) {
-  if (a.contact.act && a.contact.nv) {
+  if (a.contact.act && a.contact.nv && use_vertex_groups(a.contact.E, a.contact.nv)) {
+    hipLaunchKernelGGL(k_contact_dd, dim3(grid_for(a.contact.C)), dim3(kBlock), 0, st, a.contact, a.p, &a.s->done);
+    launch_vertex_sums(st, HvpSums{a.contact, &a.s->done}, a.contact.nv, a.contact.cverts, a.contact.v_off);
+  } else if (a.contact.act && a.contact.nv) {
     hipLaunchKernelGGL(k_contact_terms, dim3(grid_for(a.contact.E)), dim3(kBlock), 0, st, a.contact, a.p, &a.s->done);
     hipLaunchKernelGGL(k_contact_vsum, dim3(grid_for((size_t)a.contact.nv * 3)), dim3(kBlock), 0, st, a.contact,
                        &a.s->done);
