@@ -15,13 +15,14 @@
 // wave per domain, each column read contiguously.  The FP64 apply keeps the
 // reference's operation order (forward substitution column by column, which
 // subtracts in the same order as the row loop; back substitution row by row,
-// products by the wave, subtractions in order by one lane); the FP32 apply
+// products by the wave, subtractions in order by a lane per domain); the FP32 apply
 // substitutes forward by columns and backward by wave dot products.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <memory>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "elements.h"
@@ -643,122 +644,284 @@ __device__ __forceinline__ void load_block(const T* __restrict__ M, uint32_t dw,
   for (int k = 0; k < K; k++) load_col<NC, T>(M, dw, j0 + dir * k, b[k]);
 }
 
-// Forward substitution: y_j /= L_jj, then y_i -= L_ij y_j for i > j, column
-// by column; for each row the same operations in the same order as the
-// reference's row loop (schwarz.ts:262-268).
-template <int NC, int K, class T>
-__device__ __forceinline__ void forward_sub(const T* __restrict__ M, uint32_t dw, T (&y)[NC]) {
-  T cur[K][NC], nxt[K][NC];
-  load_block<NC, K, T>(M, dw, 0, 1, cur);
-  for (uint32_t jb = 0; jb < dw; jb += K) {
-    load_block<NC, K, T>(M, dw, (int)(jb + K), 1, nxt);
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-      const uint32_t j = jb + k;
-      if (j < dw) {
-        // the owner lane divides; the quotient is broadcast
-        const T yj = bcast(slot_of<NC, T>(y, j) / slot_of<NC, T>(cur[k], j), j % kWave);
-        set_slot<NC, T>(y, j, yj);
-#pragma unroll
-        for (int c = 0; c < NC; c++)
-          if (c * kWave + threadIdx.x > j) y[c] -= cur[k][c] * yj;
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < K; k++)
-#pragma unroll
-      for (int c = 0; c < NC; c++) cur[k][c] = nxt[k][c];
-  }
+// Column entries through a buffer descriptor of exactly the column's rows
+// j .. dw-1: a row outside it (a negative offset wraps to a huge one) reads 0
+// without touching memory.
+template <int N, class F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl<N>(f, std::make_integer_sequence<int, N>{});
+}
+
+using BufRsrc = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ double buf_load64(BufRsrc r, uint32_t byte_off) {
+  typedef unsigned v2u __attribute__((ext_vector_type(2)));
+  const v2u v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)byte_off, 0, 0);
+  return __builtin_bit_cast(double, v);
 }
 
 // z = A_d^-1 r on every domain, FP64, in the reference's operation order
-// (solveLocal + applySchwarz, schwarz.ts:255-309).  One wave per domain.
-// Back substitution row by row in decreasing i (:269-274): the wave forms
-// the products L_ji x_j, lane 0 subtracts them in increasing j from LDS.
-template <int NC>
-__global__ void __launch_bounds__(kWave) k_sw_apply64(SwArgs s, const double* __restrict__ r, double* z,
-                                                      const int32_t* done) {
-  constexpr int K = NC <= 3 ? 8 : 4;
-  if (done && *done) return;
-  const uint32_t d = blockIdx.x;
-  const uint32_t dv = s.size[d], dw = dv * 3;
-  const double* M = s.L + (size_t)d * tri_size(s.DW);
-  __shared__ __align__(16) double prod[NC * kWave];
-  const int lane = threadIdx.x;
-  const uint32_t* mem = s.members + (size_t)d * s.dmax;
-  double y[NC], sol[NC];
-#pragma unroll
-  for (int c = 0; c < NC; c++) {
-    const uint32_t i = c * kWave + lane;
-    y[c] = i < dw ? r[(size_t)mem[i / 3] * 3 + i % 3] : 0.0;
-    sol[c] = 0;
-  }
-  if (s.flag[d]) {
-    forward_sub<NC, K, double>(M, dw, y);
-    double cur[K][NC], nxt[K][NC];
-    load_block<NC, K, double>(M, dw, (int)dw - 1, -1, cur);
-    for (uint32_t ib = 0; ib < dw; ib += K) {
-      load_block<NC, K, double>(M, dw, (int)dw - 1 - (int)(ib + K), -1, nxt);
+// (solveLocal + applySchwarz, schwarz.ts:255-309).  One wave solves ND domains
+// side by side; row i of a domain is in lane i % 64, slot i / 64.
+//
+// Forward substitution column by column: y_j /= L_jj, then y_i -= L_ij y_j for
+// i > j, for each row the operations of the reference's row loop in its order.
+// Back substitution row by row in decreasing i (:269-274): the reference
+// subtracts L_ji x_j in increasing j, so a row's first subtraction needs the x
+// of the row just solved and dw (dw - 1) / 2 subtractions of a domain form one
+// dependent chain (18,336 for 192 rows).  That chain is the critical path:
+//   - the chains of ND domains run in one wave, lanes d, d + ND, ... all
+//     subtracting domain d's products, so they share their instructions;
+//   - a row's products go to LDS one row ahead, while the row before it is
+//     still running: only L_(i+1)i x_(i+1) is formed in the chain itself;
+//   - they are read three groups of 8 ahead; groups start at a multiple of 8,
+//     and the places at and above the diagonal hold +0 (the solution is 0
+//     there), whose subtraction changes nothing.
+// Columns are loaded K ahead (two buffers in turn).
+// Measured on 4,113 domains of 192 rows (the 512x512 fold; mean per launch of a
+// step, launches after convergence included): one domain per wave with one
+// lane subtracting and every product in the chain 669 us; here 1 domain per
+// wave 470, 2 domains 380 (K = 4: 474, fewer waves), 3 domains 395, 4 domains
+// 432 us (1,029 waves of one per SIMD: the last five make a second round).  Two
+// reads of the factor, 1.2 GB, take 234 us at the rate of a copy.
+template <int NC, int ND, int K>
+struct Sub64 {
+  uint32_t dw[ND];
+  const double* M[ND];
+  uint32_t lane;
+  bool full;  // every domain has NC * 64 rows
+  using Block = double[K][ND][NC];
+
+  // columns j0 .. j0 + K - 1, slots CLO and up
+  template <int CLO>
+  __device__ __forceinline__ void load(Block& b, uint32_t j0) const {
+    if (full) {
+      // no masks: the entries read above the diagonal belong to the column
+      // before and meet only rows that are done (forward) or zero (back)
 #pragma unroll
       for (int k = 0; k < K; k++) {
-        if (ib + k >= dw) break;
-        const uint32_t ii = dw - 1 - (ib + k);
-        // products of rows below ii (others unused); lane 0 subtracts them
-        // in increasing row order, reading them from LDS eight at a time
-        // with the next eight already requested
+        const uint32_t j = j0 + k, o = j * (NC * kWave) - j * (j - 1) / 2 - j + lane;
 #pragma unroll
-        for (int c = 0; c < NC; c++) prod[c * kWave + lane] = cur[k][c] * sol[c];
-        const double yi = bcast(slot_of<NC, double>(y, ii), ii % kWave);
-        const double lii = bcast(slot_of<NC, double>(cur[k], ii), ii % kWave);
-        __builtin_amdgcn_wave_barrier();
-        double acc = yi;
-        if (lane == 0) {
-          uint32_t j = ii + 1;
-          if ((j & 1) && j < dw) acc -= prod[j++];
-          if (j + 8 <= dw) {
-            const double2* q = reinterpret_cast<const double2*>(prod + j);
-            double2 a0 = q[0], a1 = q[1], a2 = q[2], a3 = q[3];
-            for (; j + 16 <= dw; j += 8) {
-              q = reinterpret_cast<const double2*>(prod + j + 8);
-              const double2 b0 = q[0], b1 = q[1], b2 = q[2], b3 = q[3];
-              __builtin_amdgcn_sched_barrier(0);
-              acc -= a0.x; acc -= a0.y; acc -= a1.x; acc -= a1.y;
-              acc -= a2.x; acc -= a2.y; acc -= a3.x; acc -= a3.y;
-              a0 = b0; a1 = b1; a2 = b2; a3 = b3;
-            }
-            acc -= a0.x; acc -= a0.y; acc -= a1.x; acc -= a1.y;
-            acc -= a2.x; acc -= a2.y; acc -= a3.x; acc -= a3.y;
-            j += 8;
-          }
-          for (; j < dw; j++) acc -= prod[j];
+        for (int d = 0; d < ND; d++)
+#pragma unroll
+          for (int c = CLO; c < NC; c++) b[k][d][c] = M[d][o + c * kWave];
+      }
+      return;
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      const uint32_t j = j0 + k;
+#pragma unroll
+      for (int d = 0; d < ND; d++) {
+        const bool in = j < dw[d];
+        const BufRsrc r = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<double*>(M[d] + (in ? col_off(dw[d], j) : 0)), 0, in ? (int)((dw[d] - j) * 8) : 0, 0x00027000);
+#pragma unroll
+        for (int c = CLO; c < NC; c++) b[k][d][c] = buf_load64(r, (c * kWave + lane - j) * 8u);
+      }
+    }
+  }
+};
+
+template <int NC, int ND, int K>
+__global__ void __launch_bounds__(kWave, 1) k_sw_apply64(SwArgs s, const double* __restrict__ r, double* z,
+                                                         const int32_t* done) {
+  static_assert(kWave % (2 * K) == 0, "blocks come in pairs");
+  // one domain's LDS row: room for the groups read past the end, and a stride
+  // that spreads the domains over the banks
+  constexpr int P = NC * kWave + 18;
+  if (done && *done) return;
+  __shared__ __align__(16) double prod[2][ND][P];
+  __shared__ double dia[ND][NC * kWave], sub[ND][NC * kWave], ys[ND][NC * kWave];  // L_jj, L_(j+1)j, the forward solution
+  using S64 = Sub64<NC, ND, K>;
+  S64 S;
+  const uint32_t lane = threadIdx.x;
+  S.lane = lane;
+  S.full = true;
+  uint32_t size[ND], dwm = 0;
+  double y[ND][NC], sol[ND][NC];
+#pragma unroll
+  for (int d = 0; d < ND; d++) {
+    const uint32_t dom = blockIdx.x * ND + d;
+    const bool here = dom < s.D;
+    size[d] = here ? (uint32_t)__builtin_amdgcn_readfirstlane((int)s.size[dom]) * 3 : 0;
+    // a domain on the Jacobi fallback takes no part in the substitutions
+    S.dw[d] = here && __builtin_amdgcn_readfirstlane((int)s.flag[dom]) ? size[d] : 0;
+    S.M[d] = s.L + (size_t)(here ? dom : 0) * tri_size(s.DW);
+    S.full = S.full && S.dw[d] == NC * kWave;
+    dwm = max(dwm, S.dw[d]);
+    const uint32_t* mem = s.members + (size_t)(here ? dom : 0) * s.dmax;
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      const uint32_t i = c * kWave + lane;
+      y[d][c] = i < size[d] ? r[(size_t)mem[i / 3] * 3 + i % 3] : 0.0;
+      sol[d][c] = 0;
+    }
+  }
+  typename S64::Block A, B;
+  // ---- forward
+  auto fwd = [&](const typename S64::Block& b, uint32_t j0, auto cc) __attribute__((always_inline)) {
+    constexpr int C = decltype(cc)::value;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      const uint32_t j = j0 + k, l = j % kWave;
+      if (j >= dwm) break;
+#pragma unroll
+      for (int d = 0; d < ND; d++) {
+        // every lane divides its own row, the owner's quotient is broadcast
+        const double q = y[d][C] / b[k][d][C];
+        const double yj = readlane_f64(q, l);
+        if (lane == l) {
+          dia[d][j] = b[k][d][C];
+          ys[d][j] = q;
         }
-        acc = bcast(acc, 0);
-        set_slot<NC, double>(sol, ii, acc / lii);
-        __builtin_amdgcn_wave_barrier();
-      }
+        if (lane == l + 1) sub[d][j] = b[k][d][C];
+        if constexpr (C + 1 < NC)
+          if (l == kWave - 1 && lane == 0) sub[d][j] = b[k][d][C + 1];
+        const double t = y[d][C] - b[k][d][C] * yj;
+        y[d][C] = lane > l ? t : y[d][C];
 #pragma unroll
-      for (int k = 0; k < K; k++)
-#pragma unroll
-        for (int c = 0; c < NC; c++) cur[k][c] = nxt[k][c];
-    }
-  } else {
-    // the fallback's dense product with the (diagonal) inverse, row by row
-    for (uint32_t j = 0; j < dw; j++) {
-      const double rj = r[(size_t)mem[j / 3] * 3 + j % 3];
-#pragma unroll
-      for (int c = 0; c < NC; c++) {
-        const uint32_t i = c * kWave + lane;
-        const double inv = i < dw ? M[col_off(dw, i)] : 0.0;
-        sol[c] += (j == i ? inv : 0.0) * rj;
+        for (int c = C + 1; c < NC; c++) y[d][c] -= b[k][d][c] * yj;
       }
     }
-  }
-  // out.fill(0) then out += sol for the (disjoint) members
+  };
+  if (dwm) S.template load<0>(A, 0);
+  static_for<NC>([&](auto cc) __attribute__((always_inline)) {
+    constexpr int C = decltype(cc)::value;
+    for (uint32_t lb = 0; lb < (uint32_t)kWave && C * kWave + lb < dwm; lb += 2 * K) {
+      const uint32_t j0 = C * kWave + lb;
+      S.template load<C>(B, j0 + K);
+      fwd(A, j0, cc);
+      // the next pair's first block; the last of a slot belongs to the next slot
+      if (lb + 2 * K < (uint32_t)kWave) S.template load<C>(A, j0 + 2 * K);
+      else if constexpr (C + 1 < NC) S.template load<C + 1>(A, j0 + 2 * K);
+      fwd(B, j0 + K, cc);
+    }
+  });
+  // ---- back
+  const uint32_t mine = lane % ND, groups = (dwm + 7) / 8;
+  double xprev = 0;  // x of the row solved last, domain `mine`
+  // row i from its products in LDS and xprev; all lanes take part
+  auto solve_row = [&](uint32_t i) __attribute__((always_inline)) {
+    __builtin_amdgcn_wave_barrier();
+    const double2* t = reinterpret_cast<const double2*>(prod[i & 1][mine]);
+    double2 R[3][4];
+    auto ld = [&](double2(&q)[4], uint32_t g) __attribute__((always_inline)) {
 #pragma unroll
-  for (int c = 0; c < NC; c++) {
-    const uint32_t i = c * kWave + lane;
-    if (i < dw) z[(size_t)mem[i / 3] * 3 + i % 3] = 0.0 + sol[c];
+      for (int m = 0; m < 4; m++) q[m] = t[g * 4 + m];
+    };
+    double acc;
+    auto use = [&](const double2(&q)[4]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int m = 0; m < 4; m++) {
+        acc -= q[m].x;
+        acc -= q[m].y;
+      }
+    };
+    uint32_t g = (i + 1) / 8;
+    ld(R[0], g);
+    ld(R[1], g + 1);
+    ld(R[2], g + 2);
+    const double lii = dia[mine][i];
+    acc = ys[mine][i];
+    if (i + 1 < dwm) {
+      // a domain that ends at row i has x = 0 below it
+      acc -= sub[mine][i] * xprev;
+      while (g < groups) {
+        use(R[0]);
+        ld(R[0], g + 3);
+        if (++g >= groups) break;
+        use(R[1]);
+        ld(R[1], g + 3);
+        if (++g >= groups) break;
+        use(R[2]);
+        ld(R[2], g + 3);
+        ++g;
+      }
+    }
+    return acc / lii;
+  };
+  auto back = [&](const typename S64::Block& b, uint32_t i0, auto cc) __attribute__((always_inline)) {
+    constexpr int C = decltype(cc)::value;
+#pragma unroll
+    for (int k = K - 1; k >= 0; k--) {
+      const uint32_t i = i0 + k, l = i % kWave;
+      if (i >= dwm) continue;
+      // row i's products with the rows solved so far (row i + 1 is not: +0)
+      double(&pr)[ND][P] = prod[i & 1];
+#pragma unroll
+      for (int d = 0; d < ND; d++)
+#pragma unroll
+        for (int c = C; c < NC; c++) pr[d][c * kWave + lane] = b[k][d][c] * sol[d][c];
+      if (i + 1 < dwm) {
+        const double x = solve_row(i + 1);
+        bool in = false;
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+          const double xd = readlane_f64(x, d);
+          const bool ok = i + 1 < S.dw[d];
+          sol[d][C] = ok && lane == l + 1 ? xd : sol[d][C];
+          if constexpr (C + 1 < NC) sol[d][C + 1] = ok && l == kWave - 1 && lane == 0 ? xd : sol[d][C + 1];
+          in = in || (ok && mine == (uint32_t)d);
+        }
+        xprev = in ? x : 0.0;
+      }
+    }
+  };
+  bool primed = false;
+  static_for<NC>([&](auto rc) __attribute__((always_inline)) {
+    constexpr int C = NC - 1 - decltype(rc)::value;
+    using CC = std::integral_constant<int, C>;
+    if (C * kWave >= dwm) return;
+    const uint32_t top = min(dwm - C * kWave, (uint32_t)kWave) - 1;
+    uint32_t lb = top / (2 * K) * (2 * K);  // the pair's lower block
+    if (!primed) S.template load<C>(A, C * kWave + lb + K);
+    primed = true;
+    for (;; lb -= 2 * K) {
+      const uint32_t i0 = C * kWave + lb;
+      S.template load<C>(B, i0);
+      back(A, i0 + K, CC{});
+      if (lb) S.template load<C>(A, i0 - K);
+      else if constexpr (C > 0) S.template load<C - 1>(A, i0 - K);
+      back(B, i0, CC{});
+      if (!lb) break;
+    }
+  });
+  if (dwm) {
+    const double x = solve_row(0);
+#pragma unroll
+    for (int d = 0; d < ND; d++) {
+      const double xd = readlane_f64(x, d);
+      if (S.dw[d]) sol[d][0] = lane == 0 ? xd : sol[d][0];
+    }
   }
+  static_for<ND>([&](auto dc) __attribute__((always_inline)) {
+    constexpr int d = decltype(dc)::value;
+    const uint32_t dom = blockIdx.x * ND + d;
+    if (!size[d]) return;
+    const uint32_t* mem = s.members + (size_t)dom * s.dmax;
+    if (!S.dw[d]) {
+      // the fallback's dense product with the (diagonal) inverse, row by row
+      for (uint32_t j = 0; j < size[d]; j++) {
+        const double rj = r[(size_t)mem[j / 3] * 3 + j % 3];
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+          const uint32_t i = c * kWave + lane;
+          const double inv = i < size[d] ? S.M[d][col_off(size[d], i)] : 0.0;
+          sol[d][c] += (j == i ? inv : 0.0) * rj;
+        }
+      }
+    }
+    // out.fill(0) then out += sol for the (disjoint) members
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      const uint32_t i = c * kWave + lane;
+      if (i < size[d]) z[(size_t)mem[i / 3] * 3 + i % 3] = 0.0 + sol[d][c];
+    }
+  });
 }
 
 // Row ii's entries for this lane's rows i <= ii of a triangle packed by rows.
@@ -1050,16 +1213,15 @@ void Schwarz::apply64(const double* r, double* z, const int32_t* done) {
   SchwarzImpl& S = *im_;
   if (!S.D) return;
   const SwArgs a = sw_args(S);
+#define SW_A64(C, NC, ND, K)                                                                                  \
+  case C:                                                                                                     \
+    hipLaunchKernelGGL((k_sw_apply64<NC, ND, K>), dim3((S.D + ND - 1) / ND), dim3(kWave), 0, S.st, a, r, z, done); \
+    break;
   switch ((S.DW + kWave - 1) / kWave) {
-    case 1: hipLaunchKernelGGL(k_sw_apply64<1>, dim3(S.D), dim3(kWave), 0, S.st, a, r, z, done); break;
-    case 2: hipLaunchKernelGGL(k_sw_apply64<2>, dim3(S.D), dim3(kWave), 0, S.st, a, r, z, done); break;
-    case 3: hipLaunchKernelGGL(k_sw_apply64<3>, dim3(S.D), dim3(kWave), 0, S.st, a, r, z, done); break;
-    case 4: hipLaunchKernelGGL(k_sw_apply64<4>, dim3(S.D), dim3(kWave), 0, S.st, a, r, z, done); break;
-    case 5: hipLaunchKernelGGL(k_sw_apply64<5>, dim3(S.D), dim3(kWave), 0, S.st, a, r, z, done); break;
-    case 6: hipLaunchKernelGGL(k_sw_apply64<6>, dim3(S.D), dim3(kWave), 0, S.st, a, r, z, done); break;
-    case 7: hipLaunchKernelGGL(k_sw_apply64<7>, dim3(S.D), dim3(kWave), 0, S.st, a, r, z, done); break;
-    default: hipLaunchKernelGGL(k_sw_apply64<8>, dim3(S.D), dim3(kWave), 0, S.st, a, r, z, done); break;
+    SW_A64(1, 1, 2, 4) SW_A64(2, 2, 2, 4) SW_A64(3, 3, 2, 2) SW_A64(4, 4, 2, 2) SW_A64(5, 5, 2, 2) SW_A64(6, 6, 2, 2)
+    SW_A64(7, 7, 2, 2) default: SW_A64(8, 8, 2, 2)
   }
+#undef SW_A64
   CS_LAUNCH_CHECK();
   if (S.coarse) S.coarse->apply64(r, z, done);
 }
