@@ -144,11 +144,34 @@ __device__ __forceinline__ double hinge_energy4(const double P[4][3], double res
   return 0.5 * k * dd * dd * w;
 }
 
-// FD gradient of one hinge w.r.t. vertex v (addHingeGradient, bending.ts:19-42):
-// every slot holding v is perturbed, exactly like the reference's shared copy.
+// Component i of one hinge's FD gradient w.r.t. vertex v (addHingeGradient,
+// bending.ts:19-42): every slot holding v is perturbed, exactly like the
+// reference's shared copy.
+__device__ __forceinline__ double hinge_fd(const uint32_t* vs, double P[4][3], uint32_t v, int i, double old,
+                                           double rest, double len, double asum, double k) {
+  const double eps = 1e-7;
+#pragma unroll
+  for (int s = 0; s < 4; s++)
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+      if (vs[s] == v && c == i) P[s][c] = old + eps;
+  const double ep = hinge_energy4(P, rest, len, asum, k);
+#pragma unroll
+  for (int s = 0; s < 4; s++)
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+      if (vs[s] == v && c == i) P[s][c] = old - eps;
+  const double em = hinge_energy4(P, rest, len, asum, k);
+#pragma unroll
+  for (int s = 0; s < 4; s++)
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+      if (vs[s] == v && c == i) P[s][c] = old;
+  return (ep - em) / (2 * eps);
+}
+
 __device__ __forceinline__ void hinge_grad_vertex(const DMesh& me, const double* x, uint32_t hh, uint32_t v,
                                                   double k, double* out) {
-  const double eps = 1e-7;
   uint32_t vs[4];
   double P[4][3];
 #pragma unroll
@@ -156,23 +179,9 @@ __device__ __forceinline__ void hinge_grad_vertex(const DMesh& me, const double*
     vs[s] = me.hv[(size_t)hh * 4 + s];
     ld3(x, vs[s], P[s]);
   }
-  const double rest = me.hrest[hh], len = me.hlen[hh], asum = me.hasum[hh];
 #pragma unroll
-  for (int i = 0; i < 3; i++) {
-    const double old = x[(size_t)v * 3 + i];
-#pragma unroll
-    for (int s = 0; s < 4; s++)
-      if (vs[s] == v) P[s][i] = old + eps;
-    const double ep = hinge_energy4(P, rest, len, asum, k);
-#pragma unroll
-    for (int s = 0; s < 4; s++)
-      if (vs[s] == v) P[s][i] = old - eps;
-    const double em = hinge_energy4(P, rest, len, asum, k);
-#pragma unroll
-    for (int s = 0; s < 4; s++)
-      if (vs[s] == v) P[s][i] = old;
-    out[i] = (ep - em) / (2 * eps);
-  }
+  for (int i = 0; i < 3; i++)
+    out[i] = hinge_fd(vs, P, v, i, x[(size_t)v * 3 + i], me.hrest[hh], me.hlen[hh], me.hasum[hh], k);
 }
 
 // Membrane + bending gradient at vertex v (evalInternal, fem.ts:15-54).

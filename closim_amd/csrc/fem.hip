@@ -30,10 +30,91 @@ __global__ void __launch_bounds__(kBlock) k_gradient(DMesh me, DMat mat, const d
   block_partial_dd<kBlock>(acc2, partials);
 }
 
+// The same gradient with 16 lanes per vertex: the lanes evaluate the vertex's
+// triangle corners, then the components of its hinges' gradients (two dihedral
+// energies each), and lane i < 3 adds component i in triangle and hinge order.
+// One thread evaluates 72 dihedrals of an interior vertex one after the other,
+// 84 us whatever the mesh's size up to 65,536 vertices (95 us there; 250 us for
+// 262,144, where the FP64 units are full); here the chain is 6 dihedrals, 17 us
+// for 91 as for 2,000 vertices, but lanes idle at the ends of the rounds: 116 us
+// for 65,536.  The two meet near 45,000 vertices.
+constexpr uint32_t kGradLanes = 16;
+constexpr uint32_t kGradWideMax = 32768;
+
+__global__ void __launch_bounds__(kBlock) k_gradient_wide(DMesh me, DMat mat, const double* __restrict__ x,
+                                                          const double* __restrict__ yhat, double inv_h2,
+                                                          const double* __restrict__ ceg, double* __restrict__ g,
+                                                          jsm::dd* partials) {
+  constexpr uint32_t kVerts = kBlock / kGradLanes;
+  jsm::dd acc2 = jsm::dd_zero();
+  const uint32_t sub = threadIdx.x % kGradLanes;
+  const int base = (int)(threadIdx.x % kWave - sub);
+  // uniform trip count; the groups past the last vertex take part idle
+  for (uint32_t v0 = blockIdx.x * kVerts; v0 < me.n; v0 += gridDim.x * kVerts) {
+    const uint32_t v = v0 + threadIdx.x / kGradLanes;
+    const bool valid = v < me.n;
+    double acc = 0;  // component `sub`
+    const uint32_t tb = valid ? me.vt_off[v] : 0, te = valid ? me.vt_off[v + 1] : 0;
+    for (uint32_t r = tb; r < te; r += kGradLanes) {
+      double gc[3] = {0, 0, 0};
+      if (r + sub < te) {
+        const uint32_t rec = me.vt_rec[r + sub];
+        const uint32_t t = rec >> 2;
+        double x0[3], x1[3], x2[3];
+        ld3(x, me.idx[(size_t)t * 3], x0);
+        ld3(x, me.idx[(size_t)t * 3 + 1], x1);
+        ld3(x, me.idx[(size_t)t * 3 + 2], x2);
+        tri_grad_corner(tri_state(x0, x1, x2, me.inv_dm + (size_t)t * 4), me.area[t], mat, rec & 3, gc);
+      }
+      const uint32_t cnt = min(kGradLanes, te - r);
+      for (uint32_t q = 0; q < cnt; q++) {
+        const double c0 = __shfl(gc[0], base + (int)q, kWave), c1 = __shfl(gc[1], base + (int)q, kWave),
+                     c2 = __shfl(gc[2], base + (int)q, kWave);
+        acc += sub == 0 ? c0 : sub == 1 ? c1 : c2;
+      }
+    }
+    if (mat.kb > 0) {
+      const uint32_t hb = valid ? me.vh_off[v] : 0, tasks = valid ? (me.vh_off[v + 1] - hb) * 3 : 0;
+      for (uint32_t r = 0; r < tasks; r += kGradLanes) {
+        double d = 0;
+        if (r + sub < tasks) {
+          const uint32_t hh = me.vh_rec[hb + (r + sub) / 3] >> 2;
+          const int i = (int)((r + sub) % 3);
+          uint32_t vs[4];
+          double P[4][3];
+#pragma unroll
+          for (int s = 0; s < 4; s++) {
+            vs[s] = me.hv[(size_t)hh * 4 + s];
+            ld3(x, vs[s], P[s]);
+          }
+          d = hinge_fd(vs, P, v, i, x[(size_t)v * 3 + i], me.hrest[hh], me.hlen[hh], me.hasum[hh], mat.kb);
+        }
+        const uint32_t cnt = min(kGradLanes, tasks - r);
+        for (uint32_t q = 0; q < cnt; q++) {
+          const double t = __shfl(d, base + (int)q, kWave);
+          if ((r + q) % 3 == sub) acc += t;
+        }
+      }
+    }
+    if (valid && sub < 3) {
+      const size_t i = (size_t)v * 3 + sub;
+      const double m = me.mass[v];
+      double gi = m * (x[i] - yhat[i]) * inv_h2 + acc;
+      if (ceg) gi += ceg[i];
+      if (me.pinmask[v] != 0) gi = 0;
+      g[i] = gi;
+      jsm::dd_add_prod(acc2, gi, gi);
+    }
+  }
+  block_partial_dd<kBlock>(acc2, partials);
+}
+
 void launch_gradient(hipStream_t st, const DMesh& me, const DMat& mat, const double* x, const double* yhat,
                      double inv_h2, const double* ceg, double* g, jsm::dd* partials, double* out_sumsq) {
-  const unsigned grid = red_grid(me.n);
-  hipLaunchKernelGGL(k_gradient, dim3(grid), dim3(kBlock), 0, st, me, mat, x, yhat, inv_h2, ceg, g, partials);
+  const bool wide = me.n <= kGradWideMax;
+  const unsigned grid = wide ? red_grid((size_t)me.n * kGradLanes) : red_grid(me.n);
+  hipLaunchKernelGGL(wide ? k_gradient_wide : k_gradient, dim3(grid), dim3(kBlock), 0, st, me, mat, x, yhat, inv_h2,
+                     ceg, g, partials);
   CS_LAUNCH_CHECK();
   FinishJobs f{};
   f.j[0] = FinishJob{partials, grid, FIN_DD, 0, out_sumsq};
