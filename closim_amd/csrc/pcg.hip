@@ -12,6 +12,7 @@
 // A `done` latch turns the remaining launches of a converged solve into
 // no-ops, which is exactly the reference's early return.  Block 0 records
 // decisions; every block takes them from the same merged values.
+#include "coop.h"
 #include "elements.h"
 #include "pcg.h"
 #include "schwarz.h"
@@ -27,7 +28,7 @@ __device__ __forceinline__ jsm::dd* part(const PcgArgs& a, int which) {
 
 // dd_c = kappa max(b'', 0) (J_c . p) of active contact c (distJvp,
 // contact-assembly.ts:395-414, scaled as in applyHvp :376-386).
-__device__ __forceinline__ double contact_dd(const DContactHvp& H, uint32_t ci, const double* __restrict__ p) {
+__device__ __forceinline__ double contact_dd(const DContactHvp& H, uint32_t ci, const double* p) {
   if (!H.inr[ci]) return 0.0;
   const Frozen& c = H.act[ci];
   double j;
@@ -56,19 +57,32 @@ __device__ __forceinline__ double contact_dd(const DContactHvp& H, uint32_t ci, 
   return H.coeff[ci] * j;
 }
 
+// One incident triangle corner: what does not change during a solve.
+struct HvpCorner {
+  uint32_t i0, i1, i2;
+  int corner;
+  double x0[3], x1[3], x2[3], area;
+  float inv[4];
+};
+__device__ __forceinline__ void load_corner(const PcgArgs& a, uint4 cr, HvpCorner& c) {
+  const uint32_t t = cr.w >> 2;
+  c.corner = cr.w & 3;
+  c.i0 = cr.x;
+  c.i1 = cr.y;
+  c.i2 = cr.z;
+  ld3(a.x, c.i0, c.x0); ld3(a.x, c.i1, c.x1); ld3(a.x, c.i2, c.x2);
+  const float* inv = a.me.inv_dm + (size_t)t * 4;
+  c.inv[0] = inv[0]; c.inv[1] = inv[1]; c.inv[2] = inv[2]; c.inv[3] = inv[3];
+  c.area = a.me.area[t];
+}
+
 // Contribution of one incident triangle corner to the membrane HVP at the
 // vertex: analytic, or the two gradient corners of the FD operator.
-__device__ __forceinline__ void hvp_corner(const PcgArgs& a, uint4 cr, const double* __restrict__ p, double h,
-                                           double* g0, double* g1) {
-  const DMesh& me = a.me;
-  const uint32_t t = cr.w >> 2;
-  const int corner = cr.w & 3;
-  const uint32_t i0 = cr.x, i1 = cr.y, i2 = cr.z;
-  double x0[3], x1[3], x2[3], p0[3], p1[3], p2[3];
-  ld3(a.x, i0, x0); ld3(a.x, i1, x1); ld3(a.x, i2, x2);
-  ld3(p, i0, p0); ld3(p, i1, p1); ld3(p, i2, p2);
-  const float* inv = me.inv_dm + (size_t)t * 4;
-  const double area = me.area[t];
+__device__ __forceinline__ void hvp_corner(const PcgArgs& a, const HvpCorner& c, const double* p, double h, double* g0,
+                                           double* g1) {
+  double p0[3], p1[3], p2[3];
+  ld3(p, c.i0, p0); ld3(p, c.i1, p1); ld3(p, c.i2, p2);
+  const double *x0 = c.x0, *x1 = c.x1, *x2 = c.x2;
   if (a.hvp_mode == HVP_FD) {
     // membraneHvp (fem.ts:108-130): gradients at x + h p and x - h p
     double xp0[3], xp1[3], xp2[3], xm0[3], xm1[3], xm2[3];
@@ -78,13 +92,13 @@ __device__ __forceinline__ void hvp_corner(const PcgArgs& a, uint4 cr, const dou
       xp1[i] = x1[i] + h * p1[i]; xm1[i] = x1[i] - h * p1[i];
       xp2[i] = x2[i] + h * p2[i]; xm2[i] = x2[i] - h * p2[i];
     }
-    const TriState sp = tri_state(xp0, xp1, xp2, inv);
-    tri_grad_corner(sp, area, a.mat, corner, g0);
-    const TriState sm = tri_state(xm0, xm1, xm2, inv);
-    tri_grad_corner(sm, area, a.mat, corner, g1);
+    const TriState sp = tri_state(xp0, xp1, xp2, c.inv);
+    tri_grad_corner(sp, c.area, a.mat, c.corner, g0);
+    const TriState sm = tri_state(xm0, xm1, xm2, c.inv);
+    tri_grad_corner(sm, c.area, a.mat, c.corner, g1);
   } else {
-    const TriState s = tri_state(x0, x1, x2, inv);
-    tri_hvp_corner(s, p0, p1, p2, area, a.mat, corner, g0, a.psd != 0);
+    const TriState s = tri_state(x0, x1, x2, c.inv);
+    tri_hvp_corner(s, p0, p1, p2, c.area, a.mat, c.corner, g0, a.psd != 0);
     g1[0] = g1[1] = g1[2] = 0;
   }
 }
@@ -116,8 +130,7 @@ constexpr int kLanesPerVertex = 8;
 constexpr int kVertsPerBlock = kBlock / kLanesPerVertex;
 
 // hvpFull at vertex v: M p / h^2 + H_membrane p (+ contact), unfiltered.
-// The 8 lanes of a vertex group evaluate up to 8 incident corners (and
-// contact entries) at once; lane 0 of the group adds them in list order, so
+// The 8 lanes of a vertex group evaluate up to 8 incident corners at once; lane 0 of the group adds them in list order, so
 // the sums are the reference's element-order sums bit for bit.
 __device__ __forceinline__ void hvp_vertex8(const PcgArgs& a, uint32_t v, bool valid, const double* __restrict__ p,
                                             double h, double* out) {
@@ -130,7 +143,11 @@ __device__ __forceinline__ void hvp_vertex8(const PcgArgs& a, uint32_t v, bool v
   for (uint32_t r0 = b; r0 < e; r0 += kLanesPerVertex) {
     double g0[3] = {0, 0, 0}, g1[3] = {0, 0, 0};
     const uint32_t q = r0 + sub;
-    if (q < e) hvp_corner(a, me.vt_corner[q], p, h, g0, g1);
+    if (q < e) {
+      HvpCorner c;
+      load_corner(a, me.vt_corner[q], c);
+      hvp_corner(a, c, p, h, g0, g1);
+    }
     const uint32_t cnt = min((uint32_t)kLanesPerVertex, e - r0);
     for (uint32_t j = 0; j < cnt; j++) {
 #pragma unroll
@@ -438,6 +455,287 @@ __global__ void __launch_bounds__(kBlock) k_pcg_dir(PcgArgs a, int k) {
   }
 }
 
+// ---- the whole solve in one launch (small meshes) ---------------------------
+//
+// Below a few thousand vertices an iteration of the three kernels above is
+// launches, kernel boundaries and the latency of merging partials: 25 us in
+// all (16 us of kernels) for 91 vertices as for 2,000.  Here each 8-lane group
+// keeps its vertex for the whole solve, lane i < 3 component i of r, z, p, Ap
+// and the solution in registers with the vertex's corners; only p and the
+// work-groups' sums are exchanged, three exchanges an iteration.  The
+// arithmetic is that of the kernels above (the reductions are correctly
+// rounded, whatever their tree).  Bound by the latency of three reductions
+// with their exchanges (about 2 us each) and of the FD product.  Measured per
+// iteration: 9.1 us for 91 vertices (2 work-groups), 12.6 us for 2,000 (32); a
+// step of the 13x7 strip 11.7 -> 6.1 ms, of the 20x100 strip 10.8 -> 5.0 ms.
+constexpr int kSmallBlock = 512, kSmallWaves = kSmallBlock / kWave;
+constexpr int kSmallVerts = kSmallBlock / kLanesPerVertex;  // vertices per work-group
+
+// A sum with the rounding errors of its additions summed beside it (the
+// result s + e is as if computed in twice the precision, like the
+// renormalised jsm::dd): the next addition waits for s alone, one operation,
+// where a renormalised merge waits for eleven.
+struct Sum2 {
+  double s, e;
+};
+__device__ __forceinline__ Sum2 sum2_prod(double a, double b) {
+  Sum2 r;
+  jsm::two_prod(a, b, r.s, r.e);
+  return r;
+}
+__device__ __forceinline__ Sum2 sum2_merge(Sum2 a, Sum2 b) {
+  Sum2 r;
+  double e;
+  jsm::two_sum(a.s, b.s, r.s, e);
+  r.e = (a.e + b.e) + e;
+  return r;
+}
+template <int kCtrl>
+__device__ __forceinline__ double dpp_f64(double x) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, kCtrl, 0xf, 0xf, false);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), kCtrl, 0xf, 0xf, false);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+// every lane's value plus its rotations within the row of 16 lanes
+template <int kRot>
+__device__ __forceinline__ Sum2 sum2_ror(Sum2 v) {
+  return sum2_merge(v, Sum2{dpp_f64<0x120 + kRot>(v.s), dpp_f64<0x120 + kRot>(v.e)});
+}
+__device__ __forceinline__ Sum2 sum2_xor(Sum2 v, int m) {
+  return sum2_merge(v, Sum2{__shfl_xor(v.s, m, kWave), __shfl_xor(v.e, m, kWave)});
+}
+template <int NQ>
+__device__ __forceinline__ void sum2_wave(Sum2 (&v)[NQ]) {
+#pragma unroll
+  for (int q = 0; q < NQ; q++) v[q] = sum2_ror<8>(v[q]);
+#pragma unroll
+  for (int q = 0; q < NQ; q++) v[q] = sum2_ror<4>(v[q]);
+#pragma unroll
+  for (int q = 0; q < NQ; q++) v[q] = sum2_ror<2>(v[q]);
+#pragma unroll
+  for (int q = 0; q < NQ; q++) v[q] = sum2_ror<1>(v[q]);
+#pragma unroll
+  for (int q = 0; q < NQ; q++) v[q] = sum2_xor(v[q], 16);
+#pragma unroll
+  for (int q = 0; q < NQ; q++) v[q] = sum2_xor(v[q], 32);
+}
+
+// Sums NQ values over all work-groups; every thread gets the totals.  A grid
+// barrier; with `publish`, vectors written with coop_store before it may be
+// read with plain loads after it.  False when an exchange gave up.
+template <int NQ>
+__device__ __forceinline__ bool small_sums(CoopSlots* ex, uint32_t& turn, Sum2 (&v)[NQ], double (&tot)[NQ],
+                                           bool publish) {
+  __shared__ Sum2 s_wave[NQ][kSmallWaves];
+  __shared__ double s_tot[NQ];
+  __shared__ int s_ok;
+  static_assert(kSmallWaves == 8, "the waves' sums repeat twice in a row of 16 lanes");
+  const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
+  sum2_wave(v);
+  if (lane == 0)
+#pragma unroll
+    for (int q = 0; q < NQ; q++) s_wave[q][wid] = v[q];
+  if (publish) coop_drain();
+  __syncthreads();
+  if (wid == 0) {
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+      v[q] = s_wave[q][lane % kSmallWaves];
+      v[q] = sum2_ror<1>(sum2_ror<2>(sum2_ror<4>(v[q])));
+    }
+    uint64_t mine[2 * NQ], got[2 * NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) {
+      mine[2 * q] = coop_word(v[q].s);
+      mine[2 * q + 1] = coop_word(v[q].e);
+    }
+    const bool ok = coop_exchange<2 * NQ>(ex, turn, mine, got);
+#pragma unroll
+    for (int q = 0; q < NQ; q++)
+      v[q] = Sum2{__builtin_bit_cast(double, got[2 * q]), __builtin_bit_cast(double, got[2 * q + 1])};
+    sum2_wave(v);
+    if (lane == 0) {
+#pragma unroll
+      for (int q = 0; q < NQ; q++) s_tot[q] = v[q].s + v[q].e;
+      s_ok = ok ? 1 : 0;
+    }
+    if (publish) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NQ; q++) tot[q] = s_tot[q];
+  return s_ok != 0;
+}
+
+__global__ void __launch_bounds__(kSmallBlock) k_pcg_small(PcgArgs a, CoopSlots* ex, int max_iters) {
+  const int sub = threadIdx.x % kLanesPerVertex;
+  const int base = (threadIdx.x % kWave) - sub;
+  const uint32_t v = blockIdx.x * kSmallVerts + threadIdx.x / kLanesPerVertex;
+  const bool valid = v < a.me.n, own = valid && sub < 3;
+  const size_t j = (size_t)v * 3 + sub;
+  const bool pinned = valid && a.me.pinmask[v] != 0;
+  const bool fd = a.hvp_mode == HVP_FD;
+  // the vertex's corners, 8 to a round: those of the first round stay in
+  // registers (the exchanges invalidate the caches)
+  __shared__ double s_corner[kSmallBlock][7];
+  const uint32_t cb = valid ? a.me.vt_off[v] : 0, ce = valid ? a.me.vt_off[v + 1] : 0;
+  HvpCorner first{};
+  if (cb + sub < ce) load_corner(a, a.me.vt_corner[cb + sub], first);
+  const double mass = valid ? (double)a.me.mass[v] : 0.0;
+  uint32_t turn = 0;
+  // M^-1 of the group's residual, this lane's component
+  double pre[3] = {0, 0, 0};
+  if (own) {
+    if (a.precond == PRE_BLOCK)
+      for (int i = 0; i < 3; i++) pre[i] = a.binv[(size_t)v * 9 + sub * 3 + i];
+    else
+      pre[0] = a.diag[j];
+  }
+  auto precond = [&](double r) {
+    const double r0 = __shfl(r, base, kWave), r1 = __shfl(r, base + 1, kWave), r2 = __shfl(r, base + 2, kWave);
+    if (!own || pinned) return 0.0;
+    if (a.precond == PRE_BLOCK) return pre[0] * r0 + pre[1] * r1 + pre[2] * r2;
+    return pre[0] > 1e-12 ? r / pre[0] : r;
+  };
+  const double b = own ? a.b[j] : 0.0;
+  double r = own && !pinned ? b : 0.0, sol = 0.0;
+  double z = precond(r), p = z;
+  if (own) coop_store(&a.p[j], p);
+  double rz, pp, abs_tol, residual, bnorm, pAp = 0;
+  int done = 0, iters = 0;
+  bool ok;
+  {
+    Sum2 s4[4] = {sum2_prod(b, b), sum2_prod(r, r), sum2_prod(r, z), sum2_prod(z, z)};
+    double t[4];
+    ok = small_sums<4>(ex, turn, s4, t, true);
+    bnorm = jsm::sqrt_(t[0]);
+    abs_tol = jsm::jmax(a.tol * jsm::jmax(bnorm, 1e-12), 1e-12);
+    residual = jsm::sqrt_(t[1]);
+    rz = t[2];
+    pp = t[3];
+    done = residual < abs_tol ? 2 : 0;
+  }
+  for (int k = 0; ok && !done && k < max_iters; k++) {
+    const double h = fd ? 1e-8 * (1 + jsm::sqrt_(pp)) : 0.0;
+    // as hvp_vertex8; the corners' parts go through LDS, where lane i < 3
+    // adds component i in list order
+    double acc0 = 0, acc1 = 0;
+    for (uint32_t r0 = cb; r0 < ce; r0 += kLanesPerVertex) {
+      double g0[3] = {0, 0, 0}, g1[3] = {0, 0, 0};
+      if (r0 + sub < ce) {
+        if (r0 == cb) {
+          hvp_corner(a, first, a.p, h, g0, g1);
+        } else {
+          HvpCorner c;
+          load_corner(a, a.me.vt_corner[r0 + sub], c);
+          hvp_corner(a, c, a.p, h, g0, g1);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 3; i++) {
+        s_corner[threadIdx.x][i] = g0[i];
+        s_corner[threadIdx.x][3 + i] = g1[i];
+      }
+      __builtin_amdgcn_wave_barrier();
+      if (sub < 3) {
+        const uint32_t cnt = min((uint32_t)kLanesPerVertex, ce - r0);
+        const double* g = &s_corner[threadIdx.x - sub][sub];
+        double t0[kLanesPerVertex], t1[kLanesPerVertex];
+#pragma unroll
+        for (int q = 0; q < kLanesPerVertex; q++) {
+          t0[q] = g[q * 7];
+          t1[q] = g[q * 7 + 3];
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < kLanesPerVertex; q++)
+          if (q < cnt) {
+            acc0 += t0[q];
+            acc1 += t1[q];
+          }
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    double ap = mass * p * a.inv_h2 + (fd ? (acc0 - acc1) / (2 * h) : acc0);
+    if (a.contact.act && a.contact.nv) {
+      // applyHvp per vertex: the group's lanes form 8 entries' terms at a
+      // time, added in list order
+      double cs[3] = {0, 0, 0};
+      const uint32_t eb = valid ? a.contact.v_off[v] : 0, ee = valid ? a.contact.v_off[v + 1] : 0;
+      for (uint32_t e0 = eb; e0 < ee; e0 += kLanesPerVertex) {
+        double t[3] = {0, 0, 0};
+        if (e0 + sub < ee) {
+          const uint32_t ent = a.contact.v_ent[e0 + sub];
+          if (!contact_term(a.contact, ent, contact_dd(a.contact, ent >> 3, a.p), t)) t[0] = t[1] = t[2] = 0;
+        }
+        const uint32_t cnt = min((uint32_t)kLanesPerVertex, ee - e0);
+        for (uint32_t q = 0; q < cnt; q++)
+#pragma unroll
+          for (int i = 0; i < 3; i++) cs[i] += __shfl(t[i], base + (int)q, kWave);
+      }
+      ap += sub == 0 ? cs[0] : sub == 1 ? cs[1] : cs[2];
+    }
+    if (!own || pinned) ap = 0.0;
+    {
+      Sum2 s1[1] = {sum2_prod(p, ap)};
+      double t[1];
+      ok = small_sums<1>(ex, turn, s1, t, false);
+      pAp = t[0];
+    }
+    if (!ok) break;
+    if (!(pAp > 1e-30)) {
+      done = 1;  // non-positive curvature: stop with the current x (pcg.ts:65-68)
+      iters = k;
+      break;
+    }
+    const double alpha = rz / pAp;
+    if (own && !pinned) {
+      sol = sol + alpha * p;
+      r = r - alpha * ap;
+    }
+    z = precond(r);
+    double rz_new;
+    {
+      Sum2 s2[2] = {sum2_prod(r, r), sum2_prod(r, z)};
+      double t[2];
+      ok = small_sums<2>(ex, turn, s2, t, false);
+      residual = jsm::sqrt_(t[0]);
+      rz_new = t[1];
+    }
+    if (!ok) break;
+    if (residual < abs_tol) {
+      done = 2;
+      iters = k + 1;
+      break;
+    }
+    const double beta = rz_new / rz;
+    rz = rz_new;
+    p = own && !pinned ? z + beta * p : 0.0;
+    if (own) coop_store(&a.p[j], p);
+    {
+      Sum2 s1[1] = {sum2_prod(p, p)};
+      double t[1];
+      ok = small_sums<1>(ex, turn, s1, t, true);
+      pp = t[0];
+    }
+  }
+  if (own) a.sol[j] = sol;
+  // the p.p partials of the last p, for a later HVP launch on these operands
+  if (blockIdx.x == 0)
+    for (uint32_t i = threadIdx.x; i < (a.me.n + kBlock - 1) / kBlock; i += blockDim.x)
+      part(a, PART_PP)[i] = i ? jsm::dd_zero() : jsm::dd{pp, 0.0};
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    PcgScalars* s = a.s;
+    s->rz[0] = s->rz[1] = rz;
+    s->pAp = pAp;
+    s->residual = residual;
+    s->abs_tol = abs_tol;
+    s->bnorm = bnorm;
+    s->done = done;
+    s->iters = iters;
+  }
+}
+
 unsigned pcg_grid(const PcgArgs& a) { return red_grid(a.me.n); }
 unsigned pcg_hvp_grid(const PcgArgs& a) {
   return (unsigned)std::min<size_t>(kMaxHvpBlocks, ((size_t)a.me.n + kVertsPerBlock - 1) / kVertsPerBlock);
@@ -454,6 +752,29 @@ void pcg_init(hipStream_t st, const PcgArgs& a) {
   hipLaunchKernelGGL(k_pcg_init_decide, dim3(1), dim3(kBlock), 0, st, a, pcg_grid(a));
   CS_LAUNCH_CHECK();
 }
+
+// Solves the system in one launch where that is the faster way: up to
+// kCoopMaxBlocks work-groups of 64 vertices, no Schwarz, and vertices with few
+// contacts (a vertex's entries are summed by its 8 lanes; with many,
+// k_vertex_sums gives them a work-group).  False when it was not done (another
+// path solves it, from the same inputs); *out holds the scalars otherwise.
+bool pcg_solve_small(hipStream_t st, const PcgArgs& a, int max_iters, void* exchange, PcgScalars* out) {
+  const unsigned blocks = (a.me.n + kSmallVerts - 1) / kSmallVerts;
+  if (a.precond == PRE_SCHWARZ || blocks > kCoopMaxBlocks || blocks < 1) return false;
+  if (a.contact.act && a.contact.nv && use_vertex_groups(a.contact.E, a.contact.nv)) return false;
+  CoopTicket ticket;
+  if (!ticket) return false;
+  CoopSlots* ex = static_cast<CoopSlots*>(exchange);
+  CS_HIP(hipMemsetAsync(ex, 0xff, sizeof(CoopSlots), st));
+  hipLaunchKernelGGL(k_pcg_small, dim3(blocks), dim3(kSmallBlock), 0, st, a, ex, max_iters);
+  CS_LAUNCH_CHECK();
+  uint64_t gave_up;
+  CS_HIP(hipMemcpyAsync(&gave_up, &ex->gave_up, sizeof(gave_up), hipMemcpyDeviceToHost, st));
+  CS_HIP(hipMemcpyAsync(out, a.s, sizeof(*out), hipMemcpyDeviceToHost, st));
+  CS_HIP(hipStreamSynchronize(st));
+  return gave_up == kCoopEmpty;
+}
+size_t pcg_exchange_bytes() { return sizeof(CoopSlots); }
 
 // Back-to-back HVP launches on the operands of the last solve (Ap and the
 // p.Ap partials are overwritten; the latch is cleared for the run and set after).

@@ -1,0 +1,111 @@
+"""The FP64 inner solve in one launch (meshes of up to 64 work-groups of 64
+vertices) and the gradient with 16 lanes per vertex, at the sizes where they
+can go wrong: one work-group and one vertex more or less, the largest mesh and
+the first beyond it, vertices with more corners than lanes, every
+preconditioner and Hessian operator, few and many contacts.  Equality with the
+oracle, and with the separate kernels, which CS_FLAG_TIMING selects: per-vertex
+sums keep the reference's order and the reductions are correctly rounded."""
+import numpy as np
+import pytest
+
+import oracle_ffi as O
+from closim_amd import _abi, mesh as M, scenes as S
+from closim_amd.scene import DEFAULT_MATERIAL, create_scene
+from closim_amd.solver import HipSolver
+from contact_scenes import ALL
+
+pytestmark = pytest.mark.gpu
+H = 1 / 60
+
+
+def hung(nx, ny):
+    """A sheet held by its first row, moving, its vertices jittered."""
+    pos, uv, idx = M.build_grid(nx, ny, 0.01 * nx, 0.01 * ny)
+    scene = create_scene(M.preprocess(pos, uv, idx, 0.15), DEFAULT_MATERIAL)
+    rng = np.random.default_rng(nx * 1000 + ny)
+    scene.positions += rng.uniform(-1e-4, 1e-4, scene.positions.shape)
+    scene.velocities += rng.uniform(-0.1, 0.1, scene.velocities.shape)
+    for i in range(nx + 1):
+        scene.pinned[i] = tuple(float(c) for c in scene.positions[3 * i:3 * i + 3])
+    return scene
+
+
+def fan(k):
+    """k triangles around one vertex, and a second ring: valences up to k."""
+    a = 2 * np.pi * np.arange(k) / k
+    ring = np.stack([np.cos(a), np.zeros(k), np.sin(a)], 1)
+    P = np.concatenate([[[0, 0, 0]], 0.05 * ring, 0.1 * ring]).astype(np.float32)
+    idx = []
+    for i in range(k):
+        j = (i + 1) % k
+        idx += [0, 1 + i, 1 + j, 1 + i, 1 + k + i, 1 + j, 1 + j, 1 + k + i, 1 + k + j]
+    uv = P[:, [0, 2]].copy()
+    scene = create_scene(M.preprocess(P.reshape(-1), uv.reshape(-1), np.array(idx, np.uint32), 0.15), DEFAULT_MATERIAL)
+    rng = np.random.default_rng(k)
+    scene.positions += rng.uniform(-1e-3, 1e-3, scene.positions.shape)
+    scene.pinned[1] = tuple(float(c) for c in scene.positions[3:6])
+    return scene
+
+
+def step(make, **kw):
+    g = HipSolver("fp64", **kw)
+    g.initialize(make())
+    g.step(H)
+    return g.getPositions().copy(), g.getVelocities().copy(), g.lastStats["pcg_iters"]
+
+
+def check(make, oracle=True, **kw):
+    x, v, its = step(make, **kw)
+    xs, vs, its_s = step(make, **dict(kw, flags=kw.get("flags", 0) | _abi.CS_FLAG_TIMING))
+    assert its == its_s
+    assert np.array_equal(x, xs) and np.array_equal(v, vs)
+    if oracle:
+        o = O.OracleSolver(make(), _abi.options(**kw))
+        o.step(H)
+        assert np.array_equal(x, o.getPositions()) and np.array_equal(v, o.getVelocities())
+
+
+@pytest.mark.parametrize("nx,ny", [(1, 1), (8, 6), (7, 7), (12, 4), (15, 7), (10, 11)])
+def test_sizes_match_oracle(nx, ny):
+    check(lambda: hung(nx, ny))
+
+
+@pytest.mark.parametrize("nx,ny", [(62, 64), (63, 63), (63, 64)])
+def test_largest_and_first_beyond_match_separate_kernels(nx, ny):
+    check(lambda: hung(nx, ny), oracle=False, newton_iters=3)
+
+
+@pytest.mark.parametrize("precond", [_abi.CS_PRECOND_JACOBI, _abi.CS_PRECOND_BLOCK_JACOBI])
+@pytest.mark.parametrize("hvp", [_abi.CS_HVP_FD, _abi.CS_HVP_ANALYTIC])
+def test_operators_match_oracle(precond, hvp):
+    check(lambda: hung(13, 9), precond=precond, hvp_mode=hvp)
+
+
+def test_psd_operator_matches_separate_kernels():
+    check(lambda: hung(13, 9), oracle=False, hvp_mode=_abi.CS_HVP_ANALYTIC, flags=_abi.CS_FLAG_PSD_NEWTON)
+
+
+@pytest.mark.parametrize("k", [7, 8, 9, 16, 17, 40])
+def test_high_valence_matches_oracle(k):
+    check(lambda: fan(k))
+
+
+@pytest.mark.parametrize("cap", [0, 1, 2])
+def test_iteration_caps(cap):
+    check(lambda: hung(9, 9), pcg_max_iters=cap)
+
+
+@pytest.mark.parametrize("name", ["floor", "plate", "crumpled", "stacked"])
+def test_contacts_match_oracle(name):
+    check(ALL[name])
+
+
+@pytest.mark.parametrize("nx,ny", [(180, 180), (180, 181)])
+def test_gradient_on_both_sides_of_its_rule(nx, ny):
+    # 32,761 and 32,942 vertices; one Newton iteration with one PCG iteration
+    def make():
+        return hung(nx, ny)
+    x, v, _ = step(make, newton_iters=1, pcg_max_iters=1)
+    o = O.OracleSolver(make(), _abi.options(newton_iters=1, pcg_max_iters=1))
+    o.step(H)
+    assert np.array_equal(x, o.getPositions()) and np.array_equal(v, o.getVelocities())
