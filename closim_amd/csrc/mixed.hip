@@ -5,6 +5,7 @@
 // (membrane-hvp.ts:18-108) evaluated in FP32 and FP32 reductions.  The
 // per-vertex gather over the element-ordered CSR keeps the result
 // deterministic run to run.
+#include "coop.h"
 #include "elements.h"
 #include "fem.h"
 #include "mixed.h"
@@ -367,6 +368,73 @@ __device__ __forceinline__ void k_mx_hvp_body(const MxArgs& a, int k, uint32_t b
 
 __global__ void __launch_bounds__(kBlock) k_mx_hvp(MxArgs a, int k) { k_mx_hvp_body(a, k, blockIdx.x, gridDim.x); }
 
+// A tile triangle at x: deformation, stress and weights (membrane-hvp.ts:18-45).
+// The fused multiply-adds are written out, so that every kernel that evaluates
+// a tile rounds alike.
+struct TileTri {
+  uint32_t i0, i1, i2;  // local corners
+  float ia, ib, ic, id, sc;
+  float F0[3], F1[3], S00, S11, S01;
+};
+// a b + c d, the second product rounded
+__device__ __forceinline__ float fma2(float a, float b, float c, float d) { return __builtin_fmaf(a, b, c * d); }
+__device__ __forceinline__ float dot3(const float* a, const float* b) {
+  return __builtin_fmaf(a[2], b[2], fma2(a[0], b[0], a[1], b[1]));
+}
+
+__device__ __forceinline__ TileTri tile_tri(const MxArgs& a, const TileHdr& h, uint32_t t, const float* xs) {
+#pragma clang fp contract(off)
+  const DTiles& T = a.me.tl;
+  const uint2 li = T.lidx[h.tri + t];
+  const float4 inv = T.inv[h.tri + t];
+  TileTri R;
+  R.sc = a.thick * T.area[h.tri + t];
+  R.i0 = li.x & 0xffffu; R.i1 = li.x >> 16; R.i2 = li.y;
+  R.ia = inv.x; R.ib = inv.y; R.ic = inv.z; R.id = inv.w;
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const float e1 = xs[R.i1 * 3 + k] - xs[R.i0 * 3 + k], e2 = xs[R.i2 * 3 + k] - xs[R.i0 * 3 + k];
+    R.F0[k] = fma2(R.ia, e1, R.ic, e2);
+    R.F1[k] = fma2(R.ib, e1, R.id, e2);
+  }
+  const float E00 = 0.5f * (dot3(R.F0, R.F0) - 1.f);
+  const float E11 = 0.5f * (dot3(R.F1, R.F1) - 1.f);
+  const float E01 = 0.5f * dot3(R.F0, R.F1);
+  R.S00 = fma2(a.c00, E00, a.c01, E11);
+  R.S11 = fma2(a.c01, E00, a.c11, E11);
+  R.S01 = 2.f * a.g * E01;
+  if (a.psd) stress_psd(R.S00, R.S11, R.S01);
+  return R;
+}
+// The product's nine values (three corners) for the local vector ps (:46-75).
+__device__ __forceinline__ void tile_product(const MxArgs& a, const TileTri& R, const float* ps, float* out) {
+#pragma clang fp contract(off)
+  const float *F0 = R.F0, *F1 = R.F1;
+  float dF0[3], dF1[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const float w1 = ps[R.i1 * 3 + k] - ps[R.i0 * 3 + k], w2 = ps[R.i2 * 3 + k] - ps[R.i0 * 3 + k];
+    dF0[k] = fma2(R.ia, w1, R.ic, w2);
+    dF1[k] = fma2(R.ib, w1, R.id, w2);
+  }
+  const float dE00 = dot3(F0, dF0), dE11 = dot3(F1, dF1);
+  float e = fma2(dF0[0], F1[0], F0[0], dF1[0]);
+  e = __builtin_fmaf(F0[1], dF1[1], __builtin_fmaf(dF0[1], F1[1], e));
+  e = __builtin_fmaf(F0[2], dF1[2], __builtin_fmaf(dF0[2], F1[2], e));
+  const float dE01 = 0.5f * e;
+  const float dS00 = fma2(a.c00, dE00, a.c01, dE11), dS11 = fma2(a.c01, dE00, a.c11, dE11), dS01 = 2.f * a.g * dE01;
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const float dP0 = __builtin_fmaf(F1[k], dS01, __builtin_fmaf(dF1[k], R.S01, fma2(F0[k], dS00, dF0[k], R.S00)));
+    const float dP1 = __builtin_fmaf(F1[k], dS11, __builtin_fmaf(dF1[k], R.S11, fma2(F0[k], dS01, dF0[k], R.S01)));
+    const float y1 = fma2(dP0, R.ia, dP1, R.ib);
+    const float g2 = R.sc * fma2(dP0, R.ic, dP1, R.id);
+    out[k] = -__builtin_fmaf(R.sc, y1, g2);
+    out[3 + k] = R.sc * y1;
+    out[6 + k] = g2;
+  }
+}
+
 // The same product over vertex-owner tiles: the work-group stages its local
 // vertices' x and p in LDS, evaluates every tile triangle once (all three
 // corners, membrane-hvp.ts:18-75 from x, no prepared records), then each
@@ -392,43 +460,7 @@ __device__ __forceinline__ void k_mx_hvp_tile_body(const MxArgs& a, uint32_t bid
       }
     }
     __syncthreads();
-    for (uint32_t t = threadIdx.x; t < h.n_tri; t += kBlock) {
-      const uint2 li = T.lidx[h.tri + t];
-      const float4 inv = T.inv[h.tri + t];
-      const float sc = a.thick * T.area[h.tri + t];
-      const uint32_t i0 = li.x & 0xffffu, i1 = li.x >> 16, i2 = li.y;
-      const float ia = inv.x, ib = inv.y, ic = inv.z, id = inv.w;
-      float F0[3], F1[3], dF0[3], dF1[3];
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        const float e1 = xs[i1 * 3 + k] - xs[i0 * 3 + k], e2 = xs[i2 * 3 + k] - xs[i0 * 3 + k];
-        const float w1 = ps[i1 * 3 + k] - ps[i0 * 3 + k], w2 = ps[i2 * 3 + k] - ps[i0 * 3 + k];
-        F0[k] = ia * e1 + ic * e2;
-        F1[k] = ib * e1 + id * e2;
-        dF0[k] = ia * w1 + ic * w2;
-        dF1[k] = ib * w1 + id * w2;
-      }
-      const float E00 = 0.5f * (F0[0] * F0[0] + F0[1] * F0[1] + F0[2] * F0[2] - 1.f);
-      const float E11 = 0.5f * (F1[0] * F1[0] + F1[1] * F1[1] + F1[2] * F1[2] - 1.f);
-      const float E01 = 0.5f * (F0[0] * F1[0] + F0[1] * F1[1] + F0[2] * F1[2]);
-      float S00 = a.c00 * E00 + a.c01 * E11, S11 = a.c11 * E11 + a.c01 * E00, S01 = 2.f * a.g * E01;
-      if (a.psd) stress_psd(S00, S11, S01);
-      const float dE00 = F0[0] * dF0[0] + F0[1] * dF0[1] + F0[2] * dF0[2];
-      const float dE11 = F1[0] * dF1[0] + F1[1] * dF1[1] + F1[2] * dF1[2];
-      const float dE01 = 0.5f * (dF0[0] * F1[0] + F0[0] * dF1[0] + dF0[1] * F1[1] + F0[1] * dF1[1] +
-                                 dF0[2] * F1[2] + F0[2] * dF1[2]);
-      const float dS00 = a.c00 * dE00 + a.c01 * dE11, dS11 = a.c11 * dE11 + a.c01 * dE00, dS01 = 2.f * a.g * dE01;
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        const float dP0 = dF0[k] * S00 + F0[k] * dS00 + dF1[k] * S01 + F1[k] * dS01;
-        const float dP1 = dF0[k] * S01 + F0[k] * dS01 + dF1[k] * S11 + F1[k] * dS11;
-        const float g1 = sc * (dP0 * ia + dP1 * ib);
-        const float g2 = sc * (dP0 * ic + dP1 * id);
-        out[t * 9 + k] = -(g1 + g2);
-        out[t * 9 + 3 + k] = g1;
-        out[t * 9 + 6 + k] = g2;
-      }
-    }
+    for (uint32_t t = threadIdx.x; t < h.n_tri; t += kBlock) tile_product(a, tile_tri(a, h, t, xs), ps, out + t * 9);
     __syncthreads();
     for (uint32_t o = threadIdx.x; o < h.n_own; o += kBlock) {
       const uint32_t v = T.loc[h.loc + o];
@@ -551,6 +583,218 @@ __global__ void k_mx_out(const float* sol, double* dx, size_t n3) {
   if (i < n3) dx[i] = (double)sol[i];
 }
 
+// ---- the whole solve in one launch (small meshes) ---------------------------
+//
+// An iteration of the graph's three kernels is 14 us of latency (17 with the
+// gaps) from 2,000 to 12,000 vertices: each merges the previous one's partials
+// and reads its vectors back.  Here work-group b owns tile b of the HVP (its
+// triangles' deformation and stress, and p at the tile's local vertices, stay
+// on chip) and vertices 256 b ... of the vector updates (sol, r, p in
+// registers); a tile updates p at all its local vertices itself, so that only
+// Ap, z and the partial sums are exchanged, twice an iteration.  Partial sums
+// and their trees are those of the separate kernels, so are the results.
+// Bound by the two exchanges and the LDS passes between them: 8.8 us an
+// iteration for 2,000 vertices (10 tiles), 11 us for 11,790 (55 tiles); a step of
+// the 20x100 strip 8.9 -> 4.6 ms, of a 131x90 canopy 4.8 -> 3.2 ms.
+__device__ __forceinline__ uint64_t mx_word(float a, float b) {
+  const uint64_t u = ((uint64_t)__builtin_bit_cast(uint32_t, b) << 32) | __builtin_bit_cast(uint32_t, a);
+  return u == kCoopEmpty ? 0x7fc000007fc00000ull : u;
+}
+
+// Sums two floats over the work-groups as block_partial_f and
+// merge_partials_f do over at most 64 partials: every thread gets the totals.
+__device__ __forceinline__ bool mx_sums(CoopSlots* ex, uint32_t& turn, float& a, float& b) {
+  __shared__ float s_tot[2];
+  __shared__ int s_ok;
+  coop_drain();  // this thread's part of Ap or z
+  a = block_sum_f(a);
+  b = block_sum_f(b);
+  if (threadIdx.x < kWave) {
+    const uint64_t mine[1] = {mx_word(a, b)};
+    uint64_t got[1];
+    const bool ok = coop_exchange<1>(ex, turn, mine, got);
+    float x = __builtin_bit_cast(float, (uint32_t)got[0]), y = __builtin_bit_cast(float, (uint32_t)(got[0] >> 32));
+    x = 0.f + x;
+    y = 0.f + y;
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+      x += __shfl_down(x, off, kWave);
+      y += __shfl_down(y, off, kWave);
+    }
+    if (threadIdx.x == 0) {
+      s_tot[0] = 0.f + x;
+      s_tot[1] = 0.f + y;
+      s_ok = ok ? 1 : 0;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  }
+  __syncthreads();
+  a = s_tot[0];
+  b = s_tot[1];
+  return s_ok != 0;
+}
+
+__global__ void __launch_bounds__(kBlock) k_mx_small(MxArgs a, CoopSlots* ex, int max_iters, double* dx) {
+  __shared__ float xs[kTileLoc * 3], ps[kTileLoc * 3], out[kTileTris * 9];
+  __shared__ uint8_t pin[kTileLoc];
+  constexpr int kTriSlots = (kTileTris + kBlock - 1) / kBlock, kEnt = 8;
+  const DTiles& T = a.me.tl;
+  const uint32_t tid = threadIdx.x;
+  // tile role: the tile that k_mx_hvp_tile gives this work-group
+  const uint32_t tile = (blockIdx.x % kXcds) * (gridDim.x / kXcds) + blockIdx.x / kXcds;
+  const bool tiled = tile < T.count;
+  TileHdr h{};
+  if (tiled) h = T.hdr[tile];
+  for (uint32_t l = tid; l < h.n_loc; l += kBlock) {
+    const uint32_t v = T.loc[h.loc + l];
+#pragma unroll
+    for (int k = 0; k < 3; k++) xs[l * 3 + k] = a.x[(size_t)v * 3 + k];
+    pin[l] = a.me.pinmask[v];
+  }
+  __syncthreads();
+  TileTri tri[kTriSlots];
+#pragma unroll
+  for (int q = 0; q < kTriSlots; q++)
+    if (tid + q * kBlock < h.n_tri) tri[q] = tile_tri(a, h, tid + q * kBlock, xs);
+  const bool owner = tid < h.n_own;
+  uint32_t ov = 0, e0 = 0, ecnt = 0, ent[kEnt] = {};
+  float mh = 0.f;
+  if (owner) {
+    ov = T.loc[h.loc + tid];
+    e0 = h.ent + T.off[h.off + tid];
+    ecnt = h.ent + T.off[h.off + tid + 1] - e0;
+    mh = a.me.mass[ov] * a.inv_h2;
+#pragma unroll
+    for (int q = 0; q < kEnt; q++)
+      if ((uint32_t)q < ecnt) ent[q] = T.ent[e0 + q];
+  }
+  // vector role
+  const uint32_t v = blockIdx.x * kBlock + tid;
+  const bool mine = v < a.me.n;
+  const bool pinned = mine && a.me.pinmask[v] != 0;
+  float r[3] = {0, 0, 0}, z[3] = {0, 0, 0}, p[3], sol[3] = {0, 0, 0};
+  uint32_t turn = 0;
+  float rz = 0, rr = 0;
+  if (mine) {
+    ld3f(a.r, v, r);
+    precond32(a, v, r, z);
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      if (pinned) z[i] = 0.f;
+      rz += r[i] * z[i];
+      coop_store(&a.z[(size_t)v * 3 + i], z[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++) rr += r[i] * r[i];
+  }
+#pragma unroll
+  for (int i = 0; i < 3; i++) p[i] = z[i];
+  bool ok = mx_sums(ex, turn, rz, rr);
+  float residual = sqrtf(rr), pap = 0;
+  const float abs_tol = fmaxf(a.tol * fmaxf(residual, 1e-12f), 1e-12f);
+  int done = residual < abs_tol ? 2 : 0, iters = 0;
+  float beta = 0;
+  for (int k = 0; ok && !done && k < max_iters; k++) {
+    // p at the tile's local vertices
+    for (uint32_t l = tid; l < h.n_loc; l += kBlock) {
+      const uint32_t u = T.loc[h.loc + l];
+#pragma unroll
+      for (int i = 0; i < 3; i++) {
+        const float zi = a.z[(size_t)u * 3 + i];
+        ps[l * 3 + i] = k == 0 ? zi : pin[l] ? 0.f : zi + beta * ps[l * 3 + i];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kTriSlots; q++)
+      if (tid + q * kBlock < h.n_tri) tile_product(a, tri[q], ps, out + (tid + q * kBlock) * 9);
+    __syncthreads();
+    pap = 0;
+    if (owner) {
+      float acc[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+      for (int q = 0; q < kEnt; q++)
+        if ((uint32_t)q < ecnt) {
+          const float* g = out + (ent[q] >> 2) * 9 + (ent[q] & 3) * 3;
+          acc[0] += g[0];
+          acc[1] += g[1];
+          acc[2] += g[2];
+        }
+      for (uint32_t e = kEnt; e < ecnt; e++) {
+        const uint32_t q = T.ent[e0 + e];
+        const float* g = out + (q >> 2) * 9 + (q & 3) * 3;
+        acc[0] += g[0];
+        acc[1] += g[1];
+        acc[2] += g[2];
+      }
+      const float cs[3] = {0.f, 0.f, 0.f};  // no contacts
+#pragma unroll
+      for (int i = 0; i < 3; i++) {
+        const float pv = ps[tid * 3 + i];
+        const float ap = pin[tid] ? 0.f : mh * pv + (acc[i] + cs[i]);
+        coop_store(&a.Ap[(size_t)ov * 3 + i], ap);
+        pap += pv * ap;
+      }
+    }
+    float none = 0;
+    ok = mx_sums(ex, turn, pap, none);
+    if (!ok) break;
+    if (!(pap > 1e-30f)) {
+      done = 1;
+      iters = k;
+      break;
+    }
+    const float alpha = rz / pap;
+    float rz_new = 0;
+    rr = 0;
+    if (mine) {
+#pragma unroll
+      for (int i = 0; i < 3; i++) {
+        float xi = sol[i] + alpha * p[i];
+        float ri = r[i] - alpha * a.Ap[(size_t)v * 3 + i];
+        if (pinned) { xi = 0.f; ri = 0.f; }
+        sol[i] = xi;
+        r[i] = ri;
+        rr += ri * ri;
+      }
+      precond32(a, v, r, z);
+#pragma unroll
+      for (int i = 0; i < 3; i++) {
+        if (pinned) z[i] = 0.f;
+        coop_store(&a.z[(size_t)v * 3 + i], z[i]);
+        rz_new += r[i] * z[i];
+      }
+    }
+    ok = mx_sums(ex, turn, rr, rz_new);
+    if (!ok) break;
+    residual = sqrtf(rr);
+    if (residual < abs_tol) {
+      done = 2;
+      iters = k + 1;
+      break;
+    }
+    beta = rz_new / rz;
+    rz = rz_new;
+#pragma unroll
+    for (int i = 0; i < 3; i++) p[i] = pinned ? 0.f : z[i] + beta * p[i];
+  }
+  if (!ok) return;  // the caller solves again with separate kernels
+  if (mine)
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      a.p[(size_t)v * 3 + i] = p[i];
+      dx[(size_t)v * 3 + i] = (double)sol[i];
+    }
+  if (blockIdx.x == 0 && tid == 0) {
+    MxScalars* s = a.s;
+    s->rz[0] = s->rz[1] = rz;
+    s->pAp = pap;
+    s->residual = residual;
+    s->abs_tol = abs_tol;
+    s->done = done;
+    s->iters = iters;
+  }
+}
+
 struct MixedImpl {
   hipStream_t st;
   uint32_t n;
@@ -558,6 +802,7 @@ struct MixedImpl {
   DevBuf<float> x32, d32, binv32, sol, r, z, p, Ap, partials, scan;
   DevBuf<Frozen32> act32;
   DevBuf<MxScalars> s;
+  DevBuf<CoopSlots> coop;
   MxArgs last{};
   bool has_last = false;
 };
@@ -637,6 +882,28 @@ static MxArgs prepare_args(MixedImpl& M, const MixedInputs& in, hipStream_t st) 
   return a;
 }
 
+// The solve in one launch for meshes of at most kCoopMaxBlocks tiles and
+// 256-vertex groups, without contacts or Schwarz.  The iteration count, or -1
+// when it was not done.
+static int solve_small(MixedImpl& M, const MxArgs& a, const MixedInputs& in) {
+  hipStream_t st = M.st;
+  const unsigned blocks = mx_hvp_grid(a.me);
+  if (!a.me.tl.count || blocks > kCoopMaxBlocks || mx_grid(a.me.n) > blocks) return -1;
+  CoopTicket ticket;
+  if (!ticket) return -1;
+  M.coop.alloc(1);
+  CS_HIP(hipMemsetAsync(M.coop.ptr, 0xff, sizeof(CoopSlots), st));
+  hipLaunchKernelGGL(k_mx_small, dim3(blocks), dim3(kBlock), 0, st, a, M.coop.ptr, in.max_iters, in.dx);
+  CS_LAUNCH_CHECK();
+  uint64_t gave_up;
+  MxScalars hs;
+  CS_HIP(hipMemcpyAsync(&gave_up, &M.coop.ptr->gave_up, sizeof(gave_up), hipMemcpyDeviceToHost, st));
+  CS_HIP(hipMemcpyAsync(&hs, M.s.ptr, sizeof(hs), hipMemcpyDeviceToHost, st));
+  CS_HIP(hipStreamSynchronize(st));
+  if (gave_up != kCoopEmpty) return -1;
+  return hs.done ? hs.iters : in.max_iters;
+}
+
 int MixedSolve::solve_plain(const MixedInputs& in, void (*timer)(void*, int, bool), void* ctx) {
   MixedImpl& M = *im_;
   hipStream_t st = M.st;
@@ -644,6 +911,10 @@ int MixedSolve::solve_plain(const MixedInputs& in, void (*timer)(void*, int, boo
   const MxArgs a = prepare_args(M, in, st);
   const uint32_t E = a.E;
   const dim3 g(mx_grid(n)), b(kBlock);
+  if (in.graph && !in.sw && !E) {
+    const int iters = solve_small(M, a, in);
+    if (iters >= 0) return iters;
+  }
   hipLaunchKernelGGL(k_mx_init, g, b, 0, st, a);
   if (in.sw) {
     in.sw->apply32(a.r, a.z, nullptr);
