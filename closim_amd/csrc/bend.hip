@@ -18,9 +18,10 @@ __device__ __forceinline__ void hinge_load(const DMesh& me, uint32_t h, uint32_t
 
 template <bool kHvp>
 __global__ void __launch_bounds__(kBlock) k_bend_terms(DMesh me, double k, const double* __restrict__ x,
-                                                       const double* __restrict__ p, double* __restrict__ term) {
+                                                       const double* __restrict__ p, double* __restrict__ term,
+                                                       const int32_t* done) {
   const uint32_t h = blockIdx.x * blockDim.x + threadIdx.x;
-  if (h >= me.nh) return;
+  if (h >= me.nh || (done && *done)) return;
   uint32_t v[4];
   double rest, w;
   hinge_load(me, h, v, rest, w);
@@ -65,18 +66,17 @@ __global__ void __launch_bounds__(kBlock) k_bend_vsum(DMesh me, const double* __
 void launch_bend_grad(hipStream_t st, const DMesh& me, double k, const double* x, double* term, double* out,
                       bool accumulate) {
   if (me.nh)
-    hipLaunchKernelGGL(k_bend_terms<false>, dim3(grid_for(me.nh)), dim3(kBlock), 0, st, me, k, x, nullptr, term);
+    hipLaunchKernelGGL(k_bend_terms<false>, dim3(grid_for(me.nh)), dim3(kBlock), 0, st, me, k, x, nullptr, term,
+                       nullptr);
   hipLaunchKernelGGL(k_bend_vsum, dim3(grid_for((size_t)me.n * 3)), dim3(kBlock), 0, st, me, term, out,
                      accumulate ? 1 : 0);
   CS_LAUNCH_CHECK();
 }
 
-void launch_bend_hvp(hipStream_t st, const DMesh& me, double k, const double* x, const double* p, double* term,
-                     double* out, bool accumulate) {
+void launch_bend_hvp_terms(hipStream_t st, const DMesh& me, double k, const double* x, const double* p, double* term,
+                           const int32_t* done) {
   if (me.nh)
-    hipLaunchKernelGGL(k_bend_terms<true>, dim3(grid_for(me.nh)), dim3(kBlock), 0, st, me, k, x, p, term);
-  hipLaunchKernelGGL(k_bend_vsum, dim3(grid_for((size_t)me.n * 3)), dim3(kBlock), 0, st, me, term, out,
-                     accumulate ? 1 : 0);
+    hipLaunchKernelGGL(k_bend_terms<true>, dim3(grid_for(me.nh)), dim3(kBlock), 0, st, me, k, x, p, term, done);
   CS_LAUNCH_CHECK();
 }
 

@@ -94,13 +94,15 @@ void launch_energy(hipStream_t st, const DMesh& me, const DMat& mat, const doubl
                    double h, jsm::dd* partials, double* out2);
 
 // Analytic hinge bending (bend.h; not in the reference, which differences the
-// energy): out (+)= the bending gradient, or its Hessian-vector product along
-// p, at x for hinge stiffness k; `term` holds 12 doubles per hinge.  Pinned
-// rows are zero (or left unchanged when accumulating).
+// energy): out (+)= the bending gradient at x for hinge stiffness k; `term`
+// holds 12 doubles per hinge.  Pinned rows are zero (or left unchanged when
+// accumulating).
 void launch_bend_grad(hipStream_t st, const DMesh& me, double k, const double* x, double* term, double* out,
                       bool accumulate);
-void launch_bend_hvp(hipStream_t st, const DMesh& me, double k, const double* x, const double* p, double* term,
-                     double* out, bool accumulate);
+// The per-hinge terms of its Hessian-vector product along p (summed per vertex
+// by adj_product); nothing once *done is set.
+void launch_bend_hvp_terms(hipStream_t st, const DMesh& me, double k, const double* x, const double* p, double* term,
+                           const int32_t* done);
 // Independent hinges (12 positions each) for component tests, host arrays.
 void probe_hinges(const double* X12, const double* P12, const double* rest, const double* len, const double* asum,
                   double k, uint64_t count, double* grad12, double* hvp12);

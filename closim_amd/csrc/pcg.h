@@ -83,10 +83,23 @@ double pcg_time_hvp(hipStream_t st, const PcgArgs& a, int reps);
 // blocks at x and the Jacobi diagonal.
 void launch_block_factors(hipStream_t st, const DMesh& me, const DMat& mat, const double* x, const double* diag,
                           double* binv, uint8_t* flag);
-// out = M p / h^2 + H_membrane(x) p with the analytic membrane Hessian, pins
-// zeroed (no contact): the exact part of the step adjoint's Hessian product.
-void launch_hvp64_analytic(hipStream_t st, const DMesh& me, const DMat& mat, double inv_h2, const double* x,
-                           const double* p, double* out);
+
+// Scalars of the step adjoint's block-Jacobi PCG, kept on the device so that
+// its iterations run without a host read between them.
+struct AdjPcg {
+  double rz[2];  // r.z of the current iterate and of the next, alternating with the iteration's parity
+  double pap, rr, bnorm2, rel, tol;
+  int32_t it;    // iterations taken (each with p.Ap > 0)
+  int32_t done;  // 0 running, 1 p.Ap <= 0 (not positive definite along p), 2 converged or rhs = 0
+};
+// One iteration of it on the system of `a` (x, binv, sol, r, z, p, Ap, pins,
+// partials): Ap = M p / h^2 + H_membrane(x) p (analytic) + the bending terms of
+// p (null: none), pins zeroed, and the partial sums of p.Ap; after the caller
+// has added what it adds to Ap (adj_product_dot then redoes the sums), the
+// update with its preconditioner and the next direction.
+unsigned adj_product(hipStream_t st, const PcgArgs& a, const double* bend_term, const AdjPcg* s);
+unsigned adj_product_dot(hipStream_t st, const PcgArgs& a);
+void adj_advance(hipStream_t st, const PcgArgs& a, AdjPcg* s, int cur, unsigned pap_count);
 
 // Vector helpers used by the Newton driver.
 void launch_dot(hipStream_t st, const double* a, const double* b, size_t n, jsm::dd* partials, double* out);

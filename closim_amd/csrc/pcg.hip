@@ -57,6 +57,8 @@ __device__ __forceinline__ double contact_dd(const DContactHvp& H, uint32_t ci, 
   return H.coeff[ci] * j;
 }
 
+__global__ void k_dot(const double* __restrict__ a, const double* __restrict__ b, size_t n, jsm::dd* partials);
+
 // One incident triangle corner: what does not change during a solve.
 struct HvpCorner {
   uint32_t i0, i1, i2;
@@ -347,36 +349,125 @@ __global__ void __launch_bounds__(kBlock) k_pcg_hvp(PcgArgs a, int k, unsigned p
   block_partial_dd<kBlock>(pap, part(a, PART_PAP));
 }
 
-// out = M p / h^2 + H_membrane(x) p (analytic), pins zeroed: the exact
-// membrane-and-inertia part of the Hessian for the step adjoint.
-__global__ void __launch_bounds__(kBlock) k_hvp64_analytic(PcgArgs a, const double* __restrict__ p,
-                                                           double* __restrict__ out) {
+// ---- the step adjoint's PCG -------------------------------------------------
+// Three kernels an iteration beside the hinge terms: the product with the
+// bending sums and the partial sums of p.Ap; sol, r and the preconditioner with
+// those of r.r and r.z; the stop and the next direction.  As separate products,
+// dots, finishes and vector kernels an iteration was 13 launches, 49 us of
+// them on the 128x128 sheet; now four, 33 us (the adjoint of a step 93 -> 52 ms).
+__global__ void __launch_bounds__(kBlock) k_adj_product(PcgArgs a, const double* __restrict__ term,
+                                                        const int32_t* done) {
+  if (block_latched(done)) return;
   const int sub = threadIdx.x % kLanesPerVertex;
+  const int base = (threadIdx.x % kWave) - sub;
   const uint32_t stride = gridDim.x * kVertsPerBlock;
+  jsm::dd pap = jsm::dd_zero();
   for (uint32_t v0 = blockIdx.x * kVertsPerBlock; v0 < a.me.n; v0 += stride) {
     const uint32_t v = v0 + threadIdx.x / kLanesPerVertex;
     const bool valid = v < a.me.n;
-    double o[3];
-    hvp_vertex8(a, v, valid, p, 0.0, o);
+    double o[3], s[3] = {0, 0, 0};
+    hvp_vertex8(a, v, valid, a.p, 0.0, o);
+    if (term) {
+      // the vertex's hinge terms, 8 loaded at a time, added in hinge order
+      const uint32_t hb = valid ? a.me.vh_off[v] : 0, he = valid ? a.me.vh_off[v + 1] : 0;
+      for (uint32_t r0 = hb; r0 < he; r0 += kLanesPerVertex) {
+        double t[3] = {0, 0, 0};
+        if (r0 + sub < he) {
+          const uint32_t rec = a.me.vh_rec[r0 + sub];
+          ld3(term, (rec >> 2) * 4 + (rec & 3), t);
+        }
+        const uint32_t cnt = min((uint32_t)kLanesPerVertex, he - r0);
+        for (uint32_t q = 0; q < cnt; q++)
+#pragma unroll
+          for (int i = 0; i < 3; i++) s[i] += __shfl(t[i], base + (int)q, kWave);
+      }
+    }
     if (valid && sub == 0) {
       const bool pinned = a.me.pinmask[v] != 0;
 #pragma unroll
-      for (int i = 0; i < 3; i++) out[(size_t)v * 3 + i] = pinned ? 0.0 : o[i];
+      for (int i = 0; i < 3; i++) {
+        const size_t j = (size_t)v * 3 + i;
+        const double ap = pinned ? 0.0 : term ? o[i] + s[i] : o[i];
+        a.Ap[j] = ap;
+        jsm::dd_add_prod(pap, a.p[j], ap);
+      }
     }
   }
+  block_partial_dd<kBlock>(pap, part(a, PART_PAP));
 }
 
-void launch_hvp64_analytic(hipStream_t st, const DMesh& me, const DMat& mat, double inv_h2, const double* x,
-                           const double* p, double* out) {
-  PcgArgs a{};
-  a.me = me;
-  a.mat = mat;
-  a.inv_h2 = inv_h2;
-  a.x = x;
-  a.hvp_mode = HVP_ANALYTIC;
-  a.contact.act = nullptr;
-  const unsigned g = (unsigned)std::min<size_t>(kMaxHvpBlocks, ((size_t)me.n + kVertsPerBlock - 1) / kVertsPerBlock);
-  hipLaunchKernelGGL(k_hvp64_analytic, dim3(std::max(1u, g)), dim3(kBlock), 0, st, a, p, out);
+__global__ void __launch_bounds__(kBlock) k_adj_update(PcgArgs a, AdjPcg* s, int cur, unsigned pap_count) {
+  if (block_latched(&s->done)) return;
+  const double pap = jsm::dd_value(merge_partials_dd<kBlock>(part(a, PART_PAP), pap_count));
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    s->pap = pap;
+    if (!(pap > 0)) s->done = 1;
+  }
+  if (!(pap > 0)) return;
+  const double alpha = s->rz[cur] / pap;
+  jsm::dd rr = jsm::dd_zero(), rz = jsm::dd_zero();
+  for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < a.me.n; v += gridDim.x * blockDim.x) {
+    double r3[3], z3[3];
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const size_t j = (size_t)v * 3 + i;
+      a.sol[j] += alpha * a.p[j];
+      r3[i] = a.r[j] - alpha * a.Ap[j];
+      a.r[j] = r3[i];
+      jsm::dd_add_prod(rr, r3[i], r3[i]);
+    }
+    const bool pinned = a.me.pinmask[v] != 0;
+    const double* f = a.binv + (size_t)v * 9;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      z3[i] = pinned ? 0.0 : f[3 * i] * r3[0] + f[3 * i + 1] * r3[1] + f[3 * i + 2] * r3[2];
+      a.z[(size_t)v * 3 + i] = z3[i];
+      jsm::dd_add_prod(rz, r3[i], z3[i]);
+    }
+  }
+  block_partial_dd<kBlock>(rr, part(a, PART_RR));
+  block_partial_dd<kBlock>(rz, part(a, PART_RZ));
+}
+
+__global__ void __launch_bounds__(kBlock) k_adj_dir(PcgArgs a, AdjPcg* s, int cur) {
+  if (block_latched(&s->done)) return;
+  const double rr = jsm::dd_value(merge_partials_dd<kBlock>(part(a, PART_RR), gridDim.x));
+  const double rz = jsm::dd_value(merge_partials_dd<kBlock>(part(a, PART_RZ), gridDim.x));
+  const double rel = sqrt(rr / s->bnorm2);
+  const bool stop = rel <= s->tol;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    s->rr = rr;
+    s->rz[cur ^ 1] = rz;
+    s->rel = rel;
+    s->it++;
+    if (stop) s->done = 2;
+  }
+  if (stop) return;
+  const double beta = rz / s->rz[cur];
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < (size_t)a.me.n * 3;
+       i += (size_t)gridDim.x * blockDim.x)
+    a.p[i] = a.z[i] + beta * a.p[i];
+}
+
+unsigned adj_product(hipStream_t st, const PcgArgs& a, const double* bend_term, const AdjPcg* s) {
+  const unsigned g = (unsigned)std::min<size_t>(kMaxHvpBlocks, ((size_t)a.me.n + kVertsPerBlock - 1) / kVertsPerBlock);
+  hipLaunchKernelGGL(k_adj_product, dim3(g), dim3(kBlock), 0, st, a, bend_term, &s->done);
+  CS_LAUNCH_CHECK();
+  return g;
+}
+
+unsigned adj_product_dot(hipStream_t st, const PcgArgs& a) {
+  const size_t n3 = (size_t)a.me.n * 3;
+  hipLaunchKernelGGL(k_dot, dim3(red_grid(n3)), dim3(kBlock), 0, st, a.p, a.Ap, n3,
+                     a.partials + (size_t)PART_PAP * kMaxRedBlocks);
+  CS_LAUNCH_CHECK();
+  return red_grid(n3);
+}
+
+void adj_advance(hipStream_t st, const PcgArgs& a, AdjPcg* s, int cur, unsigned pap_count) {
+  const dim3 g(red_grid(a.me.n)), b(kBlock);
+  hipLaunchKernelGGL(k_adj_update, g, b, 0, st, a, s, cur, pap_count);
+  hipLaunchKernelGGL(k_adj_dir, g, b, 0, st, a, s, cur);
   CS_LAUNCH_CHECK();
 }
 

@@ -31,15 +31,6 @@ thread_local std::string g_last_error;
 
 constexpr int kArmijoBatch = 8;  // largest batch of line-search trials evaluated before one host read
 
-// Scalars of the adjoint's block-Jacobi PCG, kept on the device so that its
-// iterations run without a host read between them.
-struct AdjPcg {
-  double rz[2];  // r.z of the current iterate and of the next, alternating with the iteration's parity
-  double pap, rr, bnorm2, rel, tol;
-  int32_t it;    // iterations taken (each with p.Ap > 0)
-  int32_t done;  // 0 running, 1 p.Ap <= 0 (not positive definite along p), 2 converged or rhs = 0
-};
-
 struct NewtonScalars {
   PcgScalars pcg;
   double grad_sumsq;
@@ -155,39 +146,6 @@ __global__ void k_adj_pcg_init(AdjPcg* a, double tol) {
   a->rel = a->bnorm2 > 0 ? 1.0 : 0.0;
 }
 
-// sol += alpha p, r -= alpha Ap, alpha = r.z / p.Ap; skipped once the solve
-// has ended or where p.Ap <= 0
-__global__ void k_adj_pcg_step(const AdjPcg* a, int cur, double* sol, double* r, const double* p, const double* ap,
-                               size_t n3) {
-  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (a->done || !(a->pap > 0)) return;
-  const double alpha = a->rz[cur] / a->pap;
-  if (i < n3) {
-    sol[i] += alpha * p[i];
-    r[i] += -alpha * ap[i];
-  }
-}
-
-// after r.r: count the iteration, its relative residual, and the stops
-__global__ void k_adj_pcg_decide(AdjPcg* a) {
-  if (a->done) return;
-  if (!(a->pap > 0)) {
-    a->done = 1;
-    return;
-  }
-  a->it++;
-  a->rel = sqrt(a->rr / a->bnorm2);
-  if (a->rel <= a->tol) a->done = 2;
-}
-
-// p = z + beta p, beta = (r.z)_next / (r.z)_current
-__global__ void k_adj_pcg_dir(const AdjPcg* a, int cur, double* p, const double* z, size_t n3) {
-  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (a->done) return;
-  const double beta = a->rz[cur ^ 1] / a->rz[cur];
-  if (i < n3) p[i] = z[i] + beta * p[i];
-}
-
 // z = B^-1 r per vertex with the block-Jacobi inverses (pins zeroed)
 __global__ void k_adj_pre_block(const double* r, const double* binv, const uint8_t* pinmask, double* z, uint32_t n) {
   const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
@@ -198,16 +156,6 @@ __global__ void k_adj_pre_block(const double* r, const double* binv, const uint8
   z[(size_t)v * 3] = pinned ? 0.0 : f[0] * r0 + f[1] * r1 + f[2] * r2;
   z[(size_t)v * 3 + 1] = pinned ? 0.0 : f[3] * r0 + f[4] * r1 + f[5] * r2;
   z[(size_t)v * 3 + 2] = pinned ? 0.0 : f[6] * r0 + f[7] * r1 + f[8] * r2;
-}
-
-__global__ void k_adj_axpy(double* y, double a, const double* x, size_t n3) {
-  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (i < n3) y[i] += a * x[i];
-}
-
-__global__ void k_adj_xpby(double* p, const double* z, double beta, size_t n3) {
-  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (i < n3) p[i] = z[i] + beta * p[i];
 }
 
 // right-hand side: dL/dx_{n+1} plus the velocity's share, free DOFs only
@@ -721,26 +669,29 @@ struct Solver {
   // gradient (the step's FD bending gradient differs from the analytic one by
   // its truncation and round-off only).
   DevBuf<double> bend_term;
-  void full_hvp(const double* base, const double* p, double* out) {
+  // A.Ap = H p and its p.Ap partial sums (their count)
+  unsigned full_hvp(const PcgArgs& A, const AdjPcg* s) {
     const size_t n3 = (size_t)n * 3;
-    launch_hvp64_analytic(st, dmesh(), dmat(), 1.0 / (hadj * hadj), base, p, out);
     const double kb = 0.5 * (mat.bend_warp + mat.bend_weft);
-    if (kb > 0 && nh) {
+    const bool bend = kb > 0 && nh;
+    if (bend) {
       bend_term.alloc((size_t)nh * 12);
-      launch_bend_hvp(st, dmesh(), kb, base, p, bend_term.ptr, out, true);
+      launch_bend_hvp_terms(st, dmesh(), kb, A.x, A.p, bend_term.ptr, &s->done);
     }
-    if (!contact) return;
+    const unsigned count = adj_product(st, A, bend ? bend_term.ptr : nullptr, s);
+    if (!contact) return count;
     // |p|_inf stays on the device (k_adj_shift / k_adj_fd_add read it)
-    launch_max_abs(st, p, n3, mpartials.ptr, &ds()->maxdx);
+    launch_max_abs(st, A.p, n3, mpartials.ptr, &ds()->maxdx);
     const double eps = 1e-6;  // metres along p / |p|_inf
     const double* pmax = &ds()->maxdx;
-    hipLaunchKernelGGL(k_adj_shift, dim3(grid_for(n3)), dim3(kBlock), 0, st, base, p, pmax, eps, adj_xs.ptr, n3);
+    hipLaunchKernelGGL(k_adj_shift, dim3(grid_for(n3)), dim3(kBlock), 0, st, A.x, A.p, pmax, eps, adj_xs.ptr, n3);
     contact_gradient(adj_xs.ptr, adj_gp.ptr);
-    hipLaunchKernelGGL(k_adj_shift, dim3(grid_for(n3)), dim3(kBlock), 0, st, base, p, pmax, -eps, adj_xs.ptr, n3);
+    hipLaunchKernelGGL(k_adj_shift, dim3(grid_for(n3)), dim3(kBlock), 0, st, A.x, A.p, pmax, -eps, adj_xs.ptr, n3);
     contact_gradient(adj_xs.ptr, adj_gm.ptr);
     hipLaunchKernelGGL(k_adj_fd_add, dim3(grid_for(n3)), dim3(kBlock), 0, st, adj_gp.ptr, adj_gm.ptr, pmax, 2 * eps,
-                       out, n3);
+                       A.Ap, n3);
     CS_LAUNCH_CHECK();
+    return adj_product_dot(st, A);
   }
 
   // the gradient term full_hvp differentiates numerically: contact alone
@@ -778,26 +729,23 @@ struct Solver {
     launch_dot(st, adj_r.ptr, adj_z.ptr, n3, partials.ptr, &A->rz[0]);
     hipLaunchKernelGGL(k_adj_pcg_init, dim3(1), dim3(1), 0, st, A, tol);
     CS_LAUNCH_CHECK();
+    PcgArgs S{};
+    S.me = dmesh();
+    S.mat = dmat();
+    S.inv_h2 = 1.0 / (hadj * hadj);
+    S.x = base;
+    S.binv = adj_binv.ptr;
+    S.sol = sol; S.r = adj_r.ptr; S.z = adj_z.ptr; S.p = adj_p.ptr; S.Ap = adj_ap.ptr;
+    S.hvp_mode = HVP_ANALYTIC;
+    S.partials = partials.ptr;
     // Iterations are enqueued in chunks and the host reads the stop flag once
     // per chunk; an iteration enqueued after the stop changes nothing (its
-    // update kernels return at once).
+    // kernels return at once).
     const int kChunk = 16;
     int cur = 0, queued = 0;
     while (queued < max_iters && read(&A->done) == 0) {
       const int m = std::min(kChunk, max_iters - queued);
-      for (int k = 0; k < m; k++, queued++, cur ^= 1) {
-        full_hvp(base, adj_p.ptr, adj_ap.ptr);
-        launch_dot(st, adj_p.ptr, adj_ap.ptr, n3, partials.ptr, &A->pap);
-        hipLaunchKernelGGL(k_adj_pcg_step, dim3(grid_for(n3)), dim3(kBlock), 0, st, A, cur, sol, adj_r.ptr,
-                           adj_p.ptr, adj_ap.ptr, n3);
-        launch_dot(st, adj_r.ptr, adj_r.ptr, n3, partials.ptr, &A->rr);
-        hipLaunchKernelGGL(k_adj_pcg_decide, dim3(1), dim3(1), 0, st, A);
-        precondition();
-        launch_dot(st, adj_r.ptr, adj_z.ptr, n3, partials.ptr, &A->rz[cur ^ 1]);
-        hipLaunchKernelGGL(k_adj_pcg_dir, dim3(grid_for(n3)), dim3(kBlock), 0, st, A, cur, adj_p.ptr, adj_z.ptr,
-                           n3);
-        CS_LAUNCH_CHECK();
-      }
+      for (int k = 0; k < m; k++, queued++, cur ^= 1) adj_advance(st, S, A, cur, full_hvp(S, A));
     }
     const AdjPcg a = read(A);
     if (iters) *iters = a.it;
