@@ -2328,6 +2328,7 @@ struct ContactImpl {
     v_off.alloc(n + 1);
     heads.alloc(n);
     klist.alloc((size_t)2 * std::max<uint32_t>(n, 1));
+    sort.block_sort = sort_setup();
     kill_lds_max = dynamic_lds_limit(reinterpret_cast<const void*>(&k_kill_run<true>));
     flow_lds_max = dynamic_lds_limit(reinterpret_cast<const void*>(&k_kill_flow));
     cverts.alloc(std::max<uint32_t>(n, 1));
@@ -2619,7 +2620,10 @@ struct ContactImpl {
                        evals.ptr, cs.ptr);
     CS_LAUNCH_CHECK();
     const size_t nent = (size_t)C * 4;
-    const bool in_tmp = radix_sort_pairs(st, ekeys.ptr, evals.ptr, ekeys_t.ptr, evals_t.ptr, nent, 0, cshift + vb, sort);
+    // the entries come out in (contact, slot) order, the low bits of the key:
+    // a stable sort on the vertex alone is enough
+    const bool in_tmp =
+        radix_sort_pairs(st, ekeys.ptr, evals.ptr, ekeys_t.ptr, evals_t.ptr, nent, cshift, cshift + vb, sort);
     const uint64_t* sk = in_tmp ? ekeys_t.ptr : ekeys.ptr;
     sync_cs();
     const uint32_t cnt = hcs->entry_count;

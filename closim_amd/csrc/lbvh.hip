@@ -92,7 +92,7 @@ constexpr Layout layout_for(uint64_t m) {
   L.keys_tmp = o; o += al256(8 * (m ? m : 1));
   L.vals = o; o += al256(4 * (m ? m : 1));
   L.vals_tmp = o; o += al256(4 * (m ? m : 1));
-  L.hist = o; o += al256(4 * 256 * ((m + 4095) / 4096 + 1));
+  L.hist = o; o += al256(4 * (radix_hist_entries(m) + 256));
   L.bsum = o; o += al256(4 * ((m + kScanBlock - 1) / kScanBlock + 1));
   L.misc = o; o += al256(sizeof(LbMisc));
   L.total = o;
