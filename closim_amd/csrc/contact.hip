@@ -53,6 +53,16 @@ struct CScalars {
   uint64_t nan_key, cross_key;
 };
 
+// zero, but no minimum and no first NaN or crossing yet
+__global__ void k_clear_counters(CScalars* cs) {
+  static_assert(sizeof(CScalars) % 8 == 0 && sizeof(CScalars) / 8 <= kBlock, "one word per thread");
+  if (threadIdx.x < sizeof(CScalars) / 8) reinterpret_cast<uint64_t*>(cs)[threadIdx.x] = 0;
+  __syncthreads();
+  if (threadIdx.x < 16) cs->mink[threadIdx.x] = ~0ull;
+  if (threadIdx.x == 16) cs->nan_key = ~0ull;
+  if (threadIdx.x == 17) cs->cross_key = ~0ull;
+}
+
 __device__ __forceinline__ void vpos(const DGeom& G, const double* x, int v, double* o) {
   if (v >= 0) {
     o[0] = x[(size_t)v * 3]; o[1] = x[(size_t)v * 3 + 1]; o[2] = x[(size_t)v * 3 + 2];
@@ -953,18 +963,18 @@ __global__ void __launch_bounds__(kBlock) k_emit_entries(const Frozen* __restric
 
 // v_ent[i] = low bits of the sorted incidence keys; v_off[u] = first entry
 // of vertex u (lower bound of u in the sorted vertex field), u in [0, n].
-__global__ void k_entry_ent(const uint64_t* __restrict__ keys, uint32_t cnt, int cshift, uint32_t* v_ent,
-                            uint32_t* ent_vtx) {
+__global__ void k_entry_ent(const uint64_t* __restrict__ keys, int cshift, uint32_t* v_ent, uint32_t* ent_vtx,
+                            const CScalars* cs) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= cnt) return;
+  if (i >= cs->entry_count) return;
   v_ent[i] = (uint32_t)(keys[i] & ((1ull << cshift) - 1));
   ent_vtx[i] = (uint32_t)(keys[i] >> cshift);
 }
 
 // Vertices that own incidence entries (order irrelevant).
-__global__ void __launch_bounds__(kBlock) k_contact_verts(const uint64_t* __restrict__ keys, uint32_t cnt, int cshift,
+__global__ void __launch_bounds__(kBlock) k_contact_verts(const uint64_t* __restrict__ keys, int cshift,
                                                           uint32_t* cverts, CScalars* cs) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, cnt = cs->entry_count;
   bool head = false;
   uint32_t u = 0;
   if (i < cnt) {
@@ -975,9 +985,9 @@ __global__ void __launch_bounds__(kBlock) k_contact_verts(const uint64_t* __rest
   if (head) cverts[k] = u;
 }
 
-__global__ void k_entry_offsets(const uint64_t* __restrict__ keys, uint32_t cnt, int cshift, uint32_t n,
-                                uint32_t* v_off) {
-  const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void k_entry_offsets(const uint64_t* __restrict__ keys, int cshift, uint32_t n, uint32_t* v_off,
+                                const CScalars* cs) {
+  const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x, cnt = cs->entry_count;
   if (u > n) return;
   uint32_t lo = 0, hi = cnt;
   while (lo < hi) {
@@ -2229,6 +2239,24 @@ struct ContactImpl {
   void sync_cs() {
     CS_HIP(hipMemcpyAsync(hcs, cs.ptr, sizeof(CScalars), hipMemcpyDeviceToHost, st));
     CS_HIP(hipStreamSynchronize(st));
+    if (red_pending) take_reds();
+  }
+
+  // The barrier energy and friction work of an energy_grad are diagnostics:
+  // they are copied out on the stream and taken at the next synchronisation
+  // instead of waiting for them.
+  DevBuf<double> ered;
+  double* hered = nullptr;  // pinned
+  bool red_pending = false;
+  void take_reds() {
+    red_pending = false;
+    diag.barrier_energy = hered[0];
+    diag.friction_work += hered[1];
+  }
+  void settle() {
+    if (!red_pending) return;
+    CS_HIP(hipStreamSynchronize(st));
+    take_reds();
   }
 
   double mink_value(int k) const {
@@ -2321,6 +2349,8 @@ struct ContactImpl {
     mkeys.alloc(m); mkeys_t.alloc(m); mvals.alloc(m); mvals_t.alloc(m);
     build_static_tree(d);
     cs.alloc(1);
+    ered.alloc(2);
+    CS_HIP(hipHostMalloc(&hered, 2 * sizeof(double)));
     ddpart.alloc(2 * kMaxRedBlocks);
     CS_HIP(hipHostMalloc(&hcs, sizeof(CScalars)));
     std::memset(hcs, 0, sizeof(CScalars));
@@ -2347,6 +2377,7 @@ struct ContactImpl {
 
   ~ContactImpl() {
     if (hcs) (void)hipHostFree(hcs);
+    if (hered) (void)hipHostFree(hered);
   }
 
   void grow_pairs(uint32_t pc, uint32_t sc) {
@@ -2368,9 +2399,11 @@ struct ContactImpl {
     ensure_sort((size_t)cap * 4);
   }
 
+  // every counter to its start in one launch (three memsets, up to two fill
+  // kernels each, were a fifth of the launches of a small step)
   void clear_counters() {
-    CS_HIP(hipMemsetAsync(cs.ptr, 0, sizeof(CScalars), st));
-    CS_HIP(hipMemsetAsync(cs.ptr->mink, 0xff, sizeof(hcs->mink), st));
+    hipLaunchKernelGGL(k_clear_counters, dim3(1), dim3(kBlock), 0, st, cs.ptr);
+    CS_LAUNCH_CHECK();
   }
 
   // Fixed hierarchy over the static triangles: unpadded exact boxes
@@ -2529,7 +2562,6 @@ struct ContactImpl {
 
   PairSrc candidate_source(const double* x, double pad) {
     clear_counters();
-    CS_HIP(hipMemsetAsync(&cs.ptr->nan_key, 0xff, 2 * sizeof(uint64_t), st));
     if (m == 0) {
       np = 0;
       nsp = 0;
@@ -2555,7 +2587,8 @@ struct ContactImpl {
     const DGeom G = geom();
     const uint32_t total = src.np + src.nsp;
     for (int attempt = 0; attempt < 3; attempt++) {
-      CS_HIP(hipMemsetAsync(&cs.ptr->pair_count, 0, 3 * sizeof(uint32_t), st));  // pair, spair, active counts
+      // pair, spair and active counts, where a traversal or an attempt wrote them
+      if (attempt || !src.filter) CS_HIP(hipMemsetAsync(&cs.ptr->pair_count, 0, 3 * sizeof(uint32_t), st));
       if (total) {
         const dim3 ag(tune_active.grid(total, st));
         if (src.filter)
@@ -2590,7 +2623,6 @@ struct ContactImpl {
                          act.ptr, anke.ptr);
       CS_LAUNCH_CHECK();
     }
-    CS_HIP(hipMemsetAsync(cs.ptr->kind_count, 0, sizeof(hcs->kind_count), st));
     if (C) hipLaunchKernelGGL(k_count_kinds, dim3(red_grid(C)), dim3(kBlock), 0, st, act.ptr, C, cs.ptr);
     build_incidence();  // syncs the scalars
     // diagnostics (contact-assembly.ts:215-219)
@@ -2604,18 +2636,18 @@ struct ContactImpl {
   int cshift = 3;
   uint32_t E = 0;   // vertex -> contact incidence entries
   uint32_t nv = 0;  // vertices with entries
+  // (kind, entry and vertex counts start at zero: candidate_source cleared them)
   void build_incidence() {
-    CS_HIP(hipMemsetAsync(v_off.ptr, 0, (size_t)(n + 1) * sizeof(uint32_t), st));
     E = 0;
     nv = 0;  // no contact vertex until the entries are rebuilt below
     if (!C) {
+      CS_HIP(hipMemsetAsync(v_off.ptr, 0, (size_t)(n + 1) * sizeof(uint32_t), st));
       sync_cs();
       return;
     }
     const int cb = bits_for(C);
     cshift = cb + 3;
     const int vb = bits_for(n) + 1;
-    CS_HIP(hipMemsetAsync(&cs.ptr->entry_count, 0, sizeof(uint32_t), st));
     hipLaunchKernelGGL(k_emit_entries, dim3(grid_for(C)), dim3(kBlock), 0, st, act.ptr, C, cshift, ekeys.ptr,
                        evals.ptr, cs.ptr);
     CS_LAUNCH_CHECK();
@@ -2625,29 +2657,23 @@ struct ContactImpl {
     const bool in_tmp =
         radix_sort_pairs(st, ekeys.ptr, evals.ptr, ekeys_t.ptr, evals_t.ptr, nent, cshift, cshift + vb, sort);
     const uint64_t* sk = in_tmp ? ekeys_t.ptr : ekeys.ptr;
-    sync_cs();
-    const uint32_t cnt = hcs->entry_count;
-    E = cnt;
-    nv = 0;
-    if (cnt) {
-      hipLaunchKernelGGL(k_entry_ent, dim3(grid_for(cnt)), dim3(kBlock), 0, st, sk, cnt, cshift, v_ent.ptr,
-                         ent_vtx.ptr);
-      hipLaunchKernelGGL(k_entry_offsets, dim3(grid_for((size_t)n + 1)), dim3(kBlock), 0, st, sk, cnt, cshift, n,
-                         v_off.ptr);
-      CS_HIP(hipMemsetAsync(&cs.ptr->nverts, 0, sizeof(uint32_t), st));
-      hipLaunchKernelGGL(k_contact_verts, dim3(grid_for(cnt)), dim3(kBlock), 0, st, sk, cnt, cshift, cverts.ptr,
-                         cs.ptr);
-      CS_HIP(hipMemsetAsync(hvsum.ptr, 0, (size_t)n * 3 * sizeof(double), st));
-      CS_LAUNCH_CHECK();
-      sync_cs();
-      nv = hcs->nverts;
-    }
+    // these read the entry count on the device, so that one host read serves all
+    hipLaunchKernelGGL(k_entry_ent, dim3(grid_for(nent)), dim3(kBlock), 0, st, sk, cshift, v_ent.ptr, ent_vtx.ptr,
+                       cs.ptr);
+    hipLaunchKernelGGL(k_entry_offsets, dim3(grid_for((size_t)n + 1)), dim3(kBlock), 0, st, sk, cshift, n, v_off.ptr,
+                       cs.ptr);
+    hipLaunchKernelGGL(k_contact_verts, dim3(grid_for(nent)), dim3(kBlock), 0, st, sk, cshift, cverts.ptr, cs.ptr);
+    CS_HIP(hipMemsetAsync(hvsum.ptr, 0, (size_t)n * 3 * sizeof(double), st));
     CS_LAUNCH_CHECK();
+    sync_cs();
+    E = hcs->entry_count;
+    nv = E ? hcs->nverts : 0;
   }
 
   CEval cev() { return CEval{inr.ptr, cg.ptr, fr.ptr, coeff.ptr}; }
 
   void energy_grad(const double* x, double* ceg, bool energies = true) {
+    settle();
     const DGeom G = geom();
     if (C) {
       hipLaunchKernelGGL(k_contact_eval, dim3(red_grid(C)), dim3(kBlock), 0, st, G, x, xstep, act.ptr, anke.ptr, C,
@@ -2655,8 +2681,8 @@ struct ContactImpl {
       CS_LAUNCH_CHECK();
       if (energies) {
         FinishJobs f{};
-        f.j[0] = FinishJob{ddpart.ptr, red_grid(C), FIN_DD, 0, &cs.ptr->red[2]};
-        f.j[1] = FinishJob{ddpart.ptr + kMaxRedBlocks, red_grid(C), FIN_DD, 0, &cs.ptr->red[3]};
+        f.j[0] = FinishJob{ddpart.ptr, red_grid(C), FIN_DD, 0, ered.ptr};
+        f.j[1] = FinishJob{ddpart.ptr + kMaxRedBlocks, red_grid(C), FIN_DD, 0, ered.ptr + 1};
         launch_finish(st, f, 2);
       }
     }
@@ -2672,9 +2698,8 @@ struct ContactImpl {
     CS_LAUNCH_CHECK();
     if (!energies) return;
     if (C) {
-      sync_cs();
-      diag.barrier_energy = hcs->red[2];
-      diag.friction_work += hcs->red[3];
+      CS_HIP(hipMemcpyAsync(hered, ered.ptr, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
+      red_pending = true;
     } else {
       diag.barrier_energy = 0;
     }
@@ -2840,6 +2865,7 @@ struct ContactImpl {
     if (count <= 0) return;
     CS_HIP(hipMemcpyAsync(hslots.data(), cs_slots.ptr, (size_t)count * sizeof(CScalars), hipMemcpyDeviceToHost, st));
     CS_HIP(hipStreamSynchronize(st));
+    if (red_pending) take_reds();
     tune_trial.collect();
     tune_ccd.collect();
   }
@@ -2953,6 +2979,7 @@ struct ContactImpl {
 ContactSystem::ContactSystem(const cs_scene_desc& d, hipStream_t st) : im_(new ContactImpl(d, st)) {}
 ContactSystem::~ContactSystem() { delete im_; }
 void ContactSystem::begin_step(const double* x0) {
+  im_->settle();
   im_->xstep = x0;
   im_->need_sort = true;
   im_->sup_valid = false;
@@ -2986,7 +3013,10 @@ void ContactSystem::friction_xstep_adjoint(const double* x, const double* lam, d
 void ContactSystem::add_rejection() { im_->diag.rejected_line_search_steps++; }
 void ContactSystem::commit(const double* x) { im_->commit(x); }
 void ContactSystem::kill_approach_velocity(const double* x, double* v) { im_->kill_approach_velocity(x, v); }
-cs_contact_diag ContactSystem::diagnostics() const { return im_->diag; }
+cs_contact_diag ContactSystem::diagnostics() const {
+  im_->settle();
+  return im_->diag;
+}
 uint64_t ContactSystem::active_count() const { return im_->C; }
 
 uint64_t ContactSystem::candidate_count() const { return im_->diag.candidate_pairs; }
