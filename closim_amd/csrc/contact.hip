@@ -787,6 +787,96 @@ __device__ __forceinline__ bool prim_separated(const Seg4& S, int kind, double d
   return all_finite && gap2 > thr * thr;
 }
 
+// The two triangles of a pair on the two sides of a slab along the line of
+// their centroids at x1 (and, with kSweep, at every time of the linear motion
+// x0 -> x1: the slab's width is the difference of a minimum and a maximum of
+// linear functions, so it is smallest at an end).  True only if every prim of
+// the pair then has a computed distance above `bound` at x1 and, with kSweep,
+// at every time, so that the reference's CCD returns Infinity (no resting
+// contact, no validated root, no sample within the thickness) wherever
+// bound > d_min.  What the argument needs of the rounded distances:
+// - edge/edge points are clamped to their edges; vertex/triangle points are
+//   inside the triangle up to the rounding of the barycentric weights, about
+//   1e-15 (e E / |n|)^2 for edges e, extent E of the pair and normal n, and no
+//   weight is 0/0, while |n| > 2.5e-4 e E: tested at x0 with a factor 4 more,
+//   and n keeps a quarter of its length on the way when the three Bernstein
+//   points of the quadratic n(t) do along n(0);
+// - the slab is wider than the bound by 1e-6 E for those weights and by 1e-9
+//   times the largest coordinates for the rounding of positions.
+// Pairs of nearby triangles of one smooth sheet, nearly all candidates, pass;
+// their swept boxes overlap, so that no box test tells them apart.
+template <bool kSweep>
+__device__ __forceinline__ bool pair_clear(const PairCorners& P, double bound) {
+  double mag = 0, E = 0;  // sum of |coordinates|; extent, 1-norm
+#pragma unroll
+  for (int s = 0; s < 6; s++) {
+    double e0 = 0, e1 = 0;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      mag += jsm::fabs_(P.x1[s][k]);
+      e1 += jsm::fabs_(P.x1[s][k] - P.x1[0][k]);
+      if (kSweep) {
+        mag += jsm::fabs_(P.x0[s][k]);
+        e0 += jsm::fabs_(P.x0[s][k] - P.x0[0][k]);
+      }
+    }
+    E = fmax(E, fmax(e0, e1));
+  }
+  E *= 2;
+  bool ok = mag <= 1e30 && E >= 1e-30;  // (false for NaN)
+  double c[3], cc = 0;
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    c[k] = (P.x1[3][k] + P.x1[4][k] + P.x1[5][k]) - (P.x1[0][k] + P.x1[1][k] + P.x1[2][k]);
+    cc += c[k] * c[k];
+  }
+  const double thr = bound * (1 + 1e-6) + (1e-6 * E + 1e-9 * mag);
+#pragma unroll
+  for (int q = kSweep ? 0 : 1; q < 2; q++) {
+    double amax = 0, bmin = __builtin_inf();  // relative to corner 0
+#pragma unroll
+    for (int s = 1; s < 6; s++) {
+      double h = 0;
+#pragma unroll
+      for (int k = 0; k < 3; k++)
+        h += c[k] * (q ? P.x1[s][k] - P.x1[0][k] : P.x0[s][k] - P.x0[0][k]);
+      if (s < 3) amax = fmax(amax, h);
+      else bmin = fmin(bmin, h);
+    }
+    const double g = bmin - amax;
+    ok = ok && g > 0 && g * g > thr * thr * cc;
+  }
+#pragma unroll
+  for (int t = 0; t < 6; t += 3) {
+    double b1[3], c1[3], n1[3], ee = 0, nn = 0;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      b1[k] = P.x1[t + 1][k] - P.x1[t][k];
+      c1[k] = P.x1[t + 2][k] - P.x1[t][k];
+    }
+    cross_v(n1, b1, c1);
+    ee = fmax(dot_v(b1, b1), dot_v(c1, c1));
+    if (kSweep) {
+      double b0[3], c0[3], n0[3], m0[3], m1[3];
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        b0[k] = P.x0[t + 1][k] - P.x0[t][k];
+        c0[k] = P.x0[t + 2][k] - P.x0[t][k];
+      }
+      cross_v(n0, b0, c0);
+      cross_v(m0, b0, c1);
+      cross_v(m1, b1, c0);
+      nn = dot_v(n0, n0);
+      ee = fmax(ee, fmax(dot_v(b0, b0), dot_v(c0, c0)));
+      ok = ok && dot_v(n1, n0) >= 0.25 * nn && 0.5 * (dot_v(m0, n0) + dot_v(m1, n0)) >= 0.25 * nn;
+    } else {
+      nn = dot_v(n1, n1);
+    }
+    ok = ok && nn >= 1e-6 * ee * E * E;
+  }
+  return ok;
+}
+
 // A CCD result of checkTrial (contact-assembly.ts:515-533): NaN marks a CCD
 // failure, a TOI in (0, 1 - 1e-9) a crossing; the smallest key of each kind
 // decides which came first in candidate order.
@@ -1949,6 +2039,51 @@ static size_t flow_lds_bytes(uint32_t nv) {
   return (size_t)nv * (sizeof(double2) + sizeof(FlowZ)) + (size_t)kFlowRing * 4 * kFlowLanes * sizeof(uint4) + 5 * kFlowLanes * 4;
 }
 
+// The prims of pair j (lanes without `on`: none).
+__device__ __forceinline__ void trial_prims(const DGeom& G, const double* __restrict__ xs,
+                                            const double* __restrict__ xt, const uint2* __restrict__ pairs,
+                                            uint32_t np, const uint2* __restrict__ spairs, uint32_t j, bool on,
+                                            double& minD, double& minT, uint2* tail, CScalars* cs) {
+  const bool stat = j >= np;
+  bool sep = true;
+  PairCorners P;
+  if (on) {
+    load_pair(G, xs, xt, stat ? spairs[j - np] : pairs[j], stat, P);
+    sep = pair_separated(P, G.d_min);
+  }
+  const int nk = stat ? 12 : 15;
+  // uniform trip count: the switch in prim_seg and the tail queue's
+  // wave-aggregated allocation see every lane
+  for (int k = 0; k < 15; k++) {
+    bool queue = false;
+    if (on && k < nk) {
+      Seg4 S;
+      prim_seg<true>(P, stat, k, S);
+      const int kind = k < (stat ? 3 : 6) ? 0 : 1;
+      const Closest c1 = kind == 0 ? closest_vt<false>(S.x1[0], S.x1[1], S.x1[2], S.x1[3])
+                                   : closest_ee<false>(S.x1[0], S.x1[1], S.x1[2], S.x1[3]);
+      // the distance only matters when it can lower this thread's minimum
+      // (or is not finite): |r|^2 above minD^2 (1 + 1e-9) rules that out
+      const double r2 = norm2(c1);
+      if (!(minD >= 1e-100 && minD <= 1e100 && r2 <= 1e200 && r2 > minD * minD * (1 + 1e-9))) {
+        const double d = jsm::hypot3(c1.rx, c1.ry, c1.rz);
+        if (d < minD) minD = d;
+        if (!jsm::isfinite_(d)) atomicOr(&cs->nonfinite, 1u);
+      }
+      if (!sep && !prim_separated(S, kind, G.d_min)) {
+        double toi;
+        if (ccd_head_fast(S, kind, G.d_min, toi)) {
+          if (toi < minT) minT = toi;  // 0 or Infinity: no crossing, no failure
+        } else {
+          queue = true;
+        }
+      }
+    }
+    const uint32_t slot = wave_alloc(queue, &cs->tail_count);
+    if (queue) tail[slot] = make_uint2(j, (uint32_t)k);
+  }
+}
+
 // checkTrial prims (contact-assembly.ts:497-535) per pair; pairs [0, np)
 // are cloth/cloth, then nsp cloth/static.  Per prim: exact distance at the
 // trial, the swept-box prefilter, then the head of the reference's CCD; the
@@ -1957,23 +2092,26 @@ static size_t flow_lds_bytes(uint32_t nv) {
 // counts go to cs->pair_count / spair_count.
 template <bool kFilter>
 __global__ void __launch_bounds__(kBlock) k_trial_pairs(DGeom G, const double* __restrict__ xs,
-                                                        const double* __restrict__ xt, double pad,
+                                                        const double* __restrict__ xt, double pad, double bound,
                                                         const uint2* __restrict__ pairs, uint32_t np,
                                                         const uint2* __restrict__ spairs, uint32_t nsp,
                                                         const double* __restrict__ sbox, uint2* tail, CScalars* cs) {
-  const uint32_t total = np + nsp;
+  __shared__ uint32_t s_q[2 * kBlock];  // pairs that are not clear of the bound
+  __shared__ uint32_t s_n;
+  const uint32_t total = np + nsp, stride = gridDim.x * blockDim.x;
   double minD = __builtin_inf(), minT = __builtin_inf();
-  for (uint32_t base = blockIdx.x * blockDim.x; base < total; base += gridDim.x * blockDim.x) {
+  if (threadIdx.x == 0) s_n = 0;
+  __syncthreads();
+  for (uint32_t base = blockIdx.x * blockDim.x; base < total; base += stride) {
     const uint32_t i = base + threadIdx.x;
     const bool stat = i >= np;
-    bool keep = false, sep = true;
-    PairCorners P;
-    uint2 pr = make_uint2(0, 0);
+    bool keep = false, todo = false;
     if (i < total) {
-      pr = stat ? spairs[i - np] : pairs[i];
+      const uint2 pr = stat ? spairs[i - np] : pairs[i];
+      PairCorners P;
       load_pair(G, xs, xt, pr, stat, P);
       keep = kFilter ? pair_keep(P, stat, pad, sbox, pr.y) : true;
-      sep = pair_separated(P, G.d_min);
+      todo = keep && !pair_clear<true>(P, bound);
     }
     if (kFilter) {
       const uint64_t mc = __ballot(keep && !stat), ms = __ballot(keep && stat);
@@ -1982,36 +2120,25 @@ __global__ void __launch_bounds__(kBlock) k_trial_pairs(DGeom G, const double* _
         if (ms) atomicAdd(&cs->spair_count, (uint32_t)__popcll(ms));
       }
     }
-    const int nk = stat ? 12 : 15;
-    // uniform trip count: the switch in prim_seg and the tail queue's
-    // wave-aggregated allocation see every lane
-    for (int k = 0; k < 15; k++) {
-      bool queue = false;
-      if (keep && k < nk) {
-        Seg4 S;
-        prim_seg<true>(P, stat, k, S);
-        const int kind = k < (stat ? 3 : 6) ? 0 : 1;
-        const Closest c1 = kind == 0 ? closest_vt<false>(S.x1[0], S.x1[1], S.x1[2], S.x1[3])
-                                     : closest_ee<false>(S.x1[0], S.x1[1], S.x1[2], S.x1[3]);
-        // the distance only matters when it can lower this thread's minimum
-        // (or is not finite): |r|^2 above minD^2 (1 + 1e-9) rules that out
-        const double r2 = norm2(c1);
-        if (!(minD >= 1e-100 && minD <= 1e100 && r2 <= 1e200 && r2 > minD * minD * (1 + 1e-9))) {
-          const double d = jsm::hypot3(c1.rx, c1.ry, c1.rz);
-          if (d < minD) minD = d;
-          if (!jsm::isfinite_(d)) atomicOr(&cs->nonfinite, 1u);
-        }
-        if (!sep && !prim_separated(S, kind, G.d_min)) {
-          double toi;
-          if (ccd_head_fast(S, kind, G.d_min, toi)) {
-            if (toi < minT) minT = toi;  // 0 or Infinity: no crossing, no failure
-          } else {
-            queue = true;
-          }
-        }
-      }
-      const uint32_t slot = wave_alloc(queue, &cs->tail_count);
-      if (queue) tail[slot] = make_uint2(i, (uint32_t)k);
+    const uint32_t at = wave_alloc(todo, &s_n);
+    if (todo) s_q[at] = i;
+    __syncthreads();
+    // whole work-groups of them, and what is left after the last pairs (at
+    // most kBlock - 1 wait from before: both together fit s_q)
+    const uint32_t n = s_n;
+    __syncthreads();  // nothing is added before every wave has read the count
+    const bool last = total - base <= stride;
+    uint32_t left = n;
+    while (left >= kBlock || (last && left)) {
+      const uint32_t take = min(left, (uint32_t)kBlock);
+      left -= take;
+      const bool on = threadIdx.x < take;
+      trial_prims(G, xs, xt, pairs, np, spairs, on ? s_q[left + threadIdx.x] : 0, on, minD, minT, tail, cs);
+    }
+    if (left != n) {
+      __syncthreads();
+      if (threadIdx.x == 0) s_n = left;
+      __syncthreads();
     }
   }
   block_min_to(minD, &cs->mink[5]);
@@ -2880,13 +3007,16 @@ struct ContactImpl {
         tail_cap = (size_t)total * 15;
         tailq.alloc(tail_cap);
       }
+      // a distance above the step's smallest so far and above d_min changes no
+      // verdict and no diagnostic
+      const double bound = std::max(diag.min_distance, prm.d_min);
       const dim3 tg(tune_trial.grid(total, st));
       if (src.filter)
-        hipLaunchKernelGGL(k_trial_pairs<true>, tg, dim3(kBlock), 0, st, G, xstep, xt, prm.d_min, src.p, src.np,
-                           src.s, src.nsp, sbox.ptr, tailq.ptr, cs.ptr);
+        hipLaunchKernelGGL(k_trial_pairs<true>, tg, dim3(kBlock), 0, st, G, xstep, xt, prm.d_min, bound, src.p,
+                           src.np, src.s, src.nsp, sbox.ptr, tailq.ptr, cs.ptr);
       else
-        hipLaunchKernelGGL(k_trial_pairs<false>, tg, dim3(kBlock), 0, st, G, xstep, xt, prm.d_min, src.p, src.np,
-                           src.s, src.nsp, sbox.ptr, tailq.ptr, cs.ptr);
+        hipLaunchKernelGGL(k_trial_pairs<false>, tg, dim3(kBlock), 0, st, G, xstep, xt, prm.d_min, bound, src.p,
+                           src.np, src.s, src.nsp, sbox.ptr, tailq.ptr, cs.ptr);
       tune_trial.after_launch(st);
       const dim3 cg(tune_ccd.grid((size_t)1 << 40, st));
       hipLaunchKernelGGL(k_trial_ccd, cg, dim3(kBlock), 0, st, G, xstep, xt, src.p, src.np, src.s, tailq.ptr,
