@@ -50,6 +50,7 @@ struct CScalars {
   uint32_t pair_count, spair_count, active_count, entry_count, nonfinite, floor_fail, nverts, kill_rounds;
   uint32_t tail_count;
   uint32_t kind_count[4];
+  uint32_t todo_count;
   uint64_t nan_key, cross_key;
 };
 
@@ -889,6 +890,18 @@ __device__ __forceinline__ void trial_toi(const DGeom& G, const Prim& q, double 
   }
 }
 
+// The waves' kept pairs into the counters, one atomic each a work-group
+// (s_kept: zero before).
+__device__ __forceinline__ void add_kept(uint32_t kept, uint32_t skept, uint32_t* s_kept, CScalars* cs) {
+  if (threadIdx.x % kWave == 0) {
+    atomicAdd(&s_kept[0], kept);
+    atomicAdd(&s_kept[1], skept);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 && s_kept[0]) atomicAdd(&cs->pair_count, s_kept[0]);
+  if (threadIdx.x == 1 && s_kept[1]) atomicAdd(&cs->spair_count, s_kept[1]);
+}
+
 // updateActiveSet (contact-assembly.ts:164-199) per pair: closest point per
 // prim at x, active when 1e-12 <= d < dHat (frozen record, sort key and
 // lagged-friction key emitted wave-aggregated); min distance over all
@@ -901,8 +914,12 @@ __global__ void __launch_bounds__(kBlock) k_active_pairs(DGeom G, const double* 
                                                          const uint2* __restrict__ spairs, uint32_t nsp,
                                                          const double* __restrict__ sbox, Frozen* rec, uint64_t* keys,
                                                          uint64_t* nkeys, uint32_t cap, CScalars* cs) {
+  __shared__ uint32_t s_kept[2];
   const uint32_t total = np + nsp;
+  uint32_t kept = 0, skept = 0;  // of the wave
   double minD = __builtin_inf();
+  if (threadIdx.x < 2) s_kept[threadIdx.x] = 0;
+  __syncthreads();
   for (uint32_t base = blockIdx.x * blockDim.x; base < total; base += gridDim.x * blockDim.x) {
     const uint32_t i = base + threadIdx.x;
     const bool stat = i >= np;
@@ -914,13 +931,8 @@ __global__ void __launch_bounds__(kBlock) k_active_pairs(DGeom G, const double* 
       load_pair(G, xs, x, pr, stat, P);
       keep = kFilter ? pair_keep(P, stat, pad, sbox, pr.y) : true;
     }
-    if (kFilter) {
-      const uint64_t mc = __ballot(keep && !stat), ms = __ballot(keep && stat);
-      if ((threadIdx.x % kWave) == 0) {
-        if (mc) atomicAdd(&cs->pair_count, (uint32_t)__popcll(mc));
-        if (ms) atomicAdd(&cs->spair_count, (uint32_t)__popcll(ms));
-      }
-    }
+    kept += (uint32_t)__popcll(__ballot(keep && !stat));
+    skept += (uint32_t)__popcll(__ballot(keep && stat));
     const int nk = stat ? 12 : 15;
     // uniform trip count so that the wave-aggregated emission sees every lane
     for (int k = 0; k < 15; k++) {
@@ -960,6 +972,7 @@ __global__ void __launch_bounds__(kBlock) k_active_pairs(DGeom G, const double* 
       }
     }
   }
+  if (kFilter) add_kept(kept, skept, s_kept, cs);
   block_min_to(minD, &cs->mink[0]);
 }
 
@@ -2039,113 +2052,122 @@ static size_t flow_lds_bytes(uint32_t nv) {
   return (size_t)nv * (sizeof(double2) + sizeof(FlowZ)) + (size_t)kFlowRing * 4 * kFlowLanes * sizeof(uint4) + 5 * kFlowLanes * 4;
 }
 
-// The prims of pair j (lanes without `on`: none).
-__device__ __forceinline__ void trial_prims(const DGeom& G, const double* __restrict__ xs,
-                                            const double* __restrict__ xt, const uint2* __restrict__ pairs,
-                                            uint32_t np, const uint2* __restrict__ spairs, uint32_t j, bool on,
-                                            double& minD, double& minT, uint2* tail, CScalars* cs) {
-  const bool stat = j >= np;
-  bool sep = true;
-  PairCorners P;
-  if (on) {
-    load_pair(G, xs, xt, stat ? spairs[j - np] : pairs[j], stat, P);
-    sep = pair_separated(P, G.d_min);
-  }
-  const int nk = stat ? 12 : 15;
-  // uniform trip count: the switch in prim_seg and the tail queue's
-  // wave-aggregated allocation see every lane
-  for (int k = 0; k < 15; k++) {
-    bool queue = false;
-    if (on && k < nk) {
-      Seg4 S;
-      prim_seg<true>(P, stat, k, S);
-      const int kind = k < (stat ? 3 : 6) ? 0 : 1;
-      const Closest c1 = kind == 0 ? closest_vt<false>(S.x1[0], S.x1[1], S.x1[2], S.x1[3])
-                                   : closest_ee<false>(S.x1[0], S.x1[1], S.x1[2], S.x1[3]);
-      // the distance only matters when it can lower this thread's minimum
-      // (or is not finite): |r|^2 above minD^2 (1 + 1e-9) rules that out
-      const double r2 = norm2(c1);
-      if (!(minD >= 1e-100 && minD <= 1e100 && r2 <= 1e200 && r2 > minD * minD * (1 + 1e-9))) {
-        const double d = jsm::hypot3(c1.rx, c1.ry, c1.rz);
-        if (d < minD) minD = d;
-        if (!jsm::isfinite_(d)) atomicOr(&cs->nonfinite, 1u);
-      }
-      if (!sep && !prim_separated(S, kind, G.d_min)) {
-        double toi;
-        if (ccd_head_fast(S, kind, G.d_min, toi)) {
-          if (toi < minT) minT = toi;  // 0 or Infinity: no crossing, no failure
-        } else {
-          queue = true;
-        }
-      }
-    }
-    const uint32_t slot = wave_alloc(queue, &cs->tail_count);
-    if (queue) tail[slot] = make_uint2(j, (uint32_t)k);
-  }
-}
-
 // checkTrial prims (contact-assembly.ts:497-535) per pair; pairs [0, np)
-// are cloth/cloth, then nsp cloth/static.  Per prim: exact distance at the
-// trial, the swept-box prefilter, then the head of the reference's CCD; the
-// few prims that need the cubic and sampling tail are queued for
-// k_trial_ccd.  With kFilter the lists are the superset and the kept pair
-// counts go to cs->pair_count / spair_count.
+// are cloth/cloth, then nsp cloth/static.  k_trial_pairs lists the pairs that
+// are not clear of `bound`; with kFilter the lists are the superset and the
+// kept pair counts go to cs->pair_count / spair_count.  It is bound by the
+// gathers of 12 positions a pair, so it holds no prim's registers and counts
+// once a work-group: an atomic a wave costs more than the pair's tests.
 template <bool kFilter>
 __global__ void __launch_bounds__(kBlock) k_trial_pairs(DGeom G, const double* __restrict__ xs,
                                                         const double* __restrict__ xt, double pad, double bound,
                                                         const uint2* __restrict__ pairs, uint32_t np,
                                                         const uint2* __restrict__ spairs, uint32_t nsp,
-                                                        const double* __restrict__ sbox, uint2* tail, CScalars* cs) {
+                                                        const double* __restrict__ sbox, uint32_t* todo, CScalars* cs) {
   __shared__ uint32_t s_q[2 * kBlock];  // pairs that are not clear of the bound
-  __shared__ uint32_t s_n;
+  __shared__ uint32_t s_n, s_at, s_kept[2];
   const uint32_t total = np + nsp, stride = gridDim.x * blockDim.x;
-  double minD = __builtin_inf(), minT = __builtin_inf();
-  if (threadIdx.x == 0) s_n = 0;
+  uint32_t kept = 0, skept = 0;  // of the wave
+  if (threadIdx.x == 0) s_n = s_kept[0] = s_kept[1] = 0;
   __syncthreads();
   for (uint32_t base = blockIdx.x * blockDim.x; base < total; base += stride) {
     const uint32_t i = base + threadIdx.x;
     const bool stat = i >= np;
-    bool keep = false, todo = false;
+    bool keep = false, open = false;
     if (i < total) {
       const uint2 pr = stat ? spairs[i - np] : pairs[i];
       PairCorners P;
       load_pair(G, xs, xt, pr, stat, P);
       keep = kFilter ? pair_keep(P, stat, pad, sbox, pr.y) : true;
-      todo = keep && !pair_clear<true>(P, bound);
+      open = keep && !pair_clear<true>(P, bound);
     }
-    if (kFilter) {
-      const uint64_t mc = __ballot(keep && !stat), ms = __ballot(keep && stat);
-      if ((threadIdx.x % kWave) == 0) {
-        if (mc) atomicAdd(&cs->pair_count, (uint32_t)__popcll(mc));
-        if (ms) atomicAdd(&cs->spair_count, (uint32_t)__popcll(ms));
-      }
-    }
-    const uint32_t at = wave_alloc(todo, &s_n);
-    if (todo) s_q[at] = i;
+    kept += (uint32_t)__popcll(__ballot(keep && !stat));
+    skept += (uint32_t)__popcll(__ballot(keep && stat));
+    const uint32_t at = wave_alloc(open, &s_n);
+    if (open) s_q[at] = i;
     __syncthreads();
-    // whole work-groups of them, and what is left after the last pairs (at
-    // most kBlock - 1 wait from before: both together fit s_q)
+    // listed when a work-group of them is there, and after the last pairs (at
+    // most kBlock - 1 wait from before, so both fit s_q)
     const uint32_t n = s_n;
     __syncthreads();  // nothing is added before every wave has read the count
-    const bool last = total - base <= stride;
-    uint32_t left = n;
-    while (left >= kBlock || (last && left)) {
-      const uint32_t take = min(left, (uint32_t)kBlock);
-      left -= take;
-      const bool on = threadIdx.x < take;
-      trial_prims(G, xs, xt, pairs, np, spairs, on ? s_q[left + threadIdx.x] : 0, on, minD, minT, tail, cs);
+    if (n >= kBlock || (total - base <= stride && n)) {
+      if (threadIdx.x == 0) {
+        s_at = atomicAdd(&cs->todo_count, n);
+        s_n = 0;
+      }
+      __syncthreads();
+      for (uint32_t k = threadIdx.x; k < n; k += kBlock) todo[s_at + k] = s_q[k];
+      __syncthreads();
     }
-    if (left != n) {
-      __syncthreads();
-      if (threadIdx.x == 0) s_n = left;
-      __syncthreads();
+  }
+  if (kFilter) add_kept(kept, skept, s_kept, cs);
+}
+
+// The prims of the listed pairs (their number is read on the device).  Per
+// prim: exact distance at the trial, the swept-box prefilter, then the head
+// of the reference's CCD; the few prims that need the cubic and sampling tail
+// are queued for k_trial_ccd.  A wave takes 64 pairs and one of kTrialParts
+// parts of their prims, so that a short list fills more of the card.
+constexpr int kTrialParts = 5;
+constexpr int kTrialPrims = 15 / kTrialParts;
+__global__ void __launch_bounds__(kBlock) k_trial_prims(DGeom G, const double* __restrict__ xs,
+                                                        const double* __restrict__ xt,
+                                                        const uint2* __restrict__ pairs, uint32_t np,
+                                                        const uint2* __restrict__ spairs,
+                                                        const uint32_t* __restrict__ todo, uint2* tail, CScalars* cs) {
+  const uint32_t cnt = cs->todo_count, items = (cnt + kWave - 1) / kWave * kTrialParts;
+  double minD = __builtin_inf(), minT = __builtin_inf();
+  constexpr uint32_t kWaves = kBlock / kWave;
+  const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWaves + threadIdx.x / kWave));
+  for (uint32_t w = first; w < items; w += gridDim.x * kWaves) {
+    const uint32_t t = w / kTrialParts * kWave + threadIdx.x % kWave;
+    const int k0 = (int)(w % kTrialParts) * kTrialPrims;
+    const bool on = t < cnt;
+    const uint32_t j = on ? todo[t] : 0;
+    const bool stat = j >= np;
+    bool sep = true;
+    PairCorners P;
+    if (on) {
+      load_pair(G, xs, xt, stat ? spairs[j - np] : pairs[j], stat, P);
+      sep = pair_separated(P, G.d_min);
+    }
+    const int nk = stat ? 12 : 15;
+    // uniform trip count: the switch in prim_seg and the tail queue's
+    // wave-aggregated allocation see every lane
+    for (int k = k0; k < k0 + kTrialPrims; k++) {
+      bool queue = false;
+      if (on && k < nk) {
+        Seg4 S;
+        prim_seg<true>(P, stat, k, S);
+        const int kind = k < (stat ? 3 : 6) ? 0 : 1;
+        const Closest c1 = kind == 0 ? closest_vt<false>(S.x1[0], S.x1[1], S.x1[2], S.x1[3])
+                                     : closest_ee<false>(S.x1[0], S.x1[1], S.x1[2], S.x1[3]);
+        // the distance only matters when it can lower this thread's minimum
+        // (or is not finite): |r|^2 above minD^2 (1 + 1e-9) rules that out
+        const double r2 = norm2(c1);
+        if (!(minD >= 1e-100 && minD <= 1e100 && r2 <= 1e200 && r2 > minD * minD * (1 + 1e-9))) {
+          const double d = jsm::hypot3(c1.rx, c1.ry, c1.rz);
+          if (d < minD) minD = d;
+          if (!jsm::isfinite_(d)) atomicOr(&cs->nonfinite, 1u);
+        }
+        if (!sep && !prim_separated(S, kind, G.d_min)) {
+          double toi;
+          if (ccd_head_fast(S, kind, G.d_min, toi)) {
+            if (toi < minT) minT = toi;  // 0 or Infinity: no crossing, no failure
+          } else {
+            queue = true;
+          }
+        }
+      }
+      const uint32_t slot = wave_alloc(queue, &cs->tail_count);
+      if (queue) tail[slot] = make_uint2(j, (uint32_t)k);
     }
   }
   block_min_to(minD, &cs->mink[5]);
   block_min_to(minT, &cs->mink[6]);
 }
 
-// The CCD tail (cubic roots, sampled fallback) of the prims k_trial_pairs
+// The CCD tail (cubic roots, sampled fallback) of the prims k_trial_prims
 // queued; the queue length is read on the device.
 __global__ void __launch_bounds__(kBlock) k_trial_ccd(DGeom G, const double* __restrict__ xs,
                                                       const double* __restrict__ xt,
@@ -2312,6 +2334,7 @@ struct ContactImpl {
   DevBuf<uint2> pairs, spairs;
   DevBuf<uint2> tailq;  // (pair, prim) items for the CCD tail
   size_t tail_cap = 0;
+  DevBuf<uint32_t> todo;  // pairs whose prims a trial evaluates
   uint32_t pair_cap = 0, spair_cap = 0, np = 0, nsp = 0;
   // active set
   DevBuf<Frozen> rec, act;
@@ -3006,6 +3029,7 @@ struct ContactImpl {
       if ((size_t)total * 15 > tail_cap) {
         tail_cap = (size_t)total * 15;
         tailq.alloc(tail_cap);
+        todo.alloc(total);
       }
       // a distance above the step's smallest so far and above d_min changes no
       // verdict and no diagnostic
@@ -3013,11 +3037,14 @@ struct ContactImpl {
       const dim3 tg(tune_trial.grid(total, st));
       if (src.filter)
         hipLaunchKernelGGL(k_trial_pairs<true>, tg, dim3(kBlock), 0, st, G, xstep, xt, prm.d_min, bound, src.p,
-                           src.np, src.s, src.nsp, sbox.ptr, tailq.ptr, cs.ptr);
+                           src.np, src.s, src.nsp, sbox.ptr, todo.ptr, cs.ptr);
       else
         hipLaunchKernelGGL(k_trial_pairs<false>, tg, dim3(kBlock), 0, st, G, xstep, xt, prm.d_min, bound, src.p,
-                           src.np, src.s, src.nsp, sbox.ptr, tailq.ptr, cs.ptr);
+                           src.np, src.s, src.nsp, sbox.ptr, todo.ptr, cs.ptr);
       tune_trial.after_launch(st);
+      const dim3 pg(std::min(grid_for((size_t)total * kTrialParts), 2048u));
+      hipLaunchKernelGGL(k_trial_prims, pg, dim3(kBlock), 0, st, G, xstep, xt, src.p, src.np, src.s, todo.ptr,
+                         tailq.ptr, cs.ptr);
       const dim3 cg(tune_ccd.grid((size_t)1 << 40, st));
       hipLaunchKernelGGL(k_trial_ccd, cg, dim3(kBlock), 0, st, G, xstep, xt, src.p, src.np, src.s, tailq.ptr,
                          cs.ptr);
