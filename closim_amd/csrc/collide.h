@@ -211,6 +211,7 @@ __device__ __forceinline__ double stencil_dev(const Seg4& S) {
   return dev;
 }
 
+template <bool kDist>
 __device__ __forceinline__ Closest ee_at(const double* a0, const double* da, const double* b0, const double* db,
                                          const double* c0, const double* dc, const double* d0, const double* dd,
                                          double t);
@@ -231,7 +232,7 @@ __device__ inline bool ccd_head(const Seg4& S, int kind, double thickness, doubl
       c0[i] = S.x0[2][i]; dc[i] = S.x1[2][i] - S.x0[2][i];
       e0[i] = S.x0[3][i]; de[i] = S.x1[3][i] - S.x0[3][i];
     }
-    d0 = ee_at(a0, da, b0, db, c0, dc, e0, de, 0).dist;
+    d0 = ee_at<true>(a0, da, b0, db, c0, dc, e0, de, 0).dist;
   }
   if (d0 <= thickness) {
     toi = 0;
@@ -287,12 +288,40 @@ __device__ inline bool ccd_head_fast(const Seg4& S, int kind, double thickness, 
   return ccd_head(S, kind, thickness, toi);
 }
 
-// vtCCD() ccd-vt.ts:20-115; slots 0..3 = p, a, b, c.
-__device__ inline double vt_ccd(const Seg4& S, double thickness) {
-  const double d0 = closest_vt(S.x0[0], S.x0[1], S.x0[2], S.x0[3]).dist;
-  if (d0 <= thickness) return 0;
-  const double dev = stencil_dev(S);
-  if (d0 - 4 * dev > thickness) return __builtin_inf();
+// The distance of a closest point where it may be at most `thickness`, or
+// Infinity where |r|^2 rules that out (the hypot of the reference is within a
+// few ulp of |r|).  Both CCD routines only ask for distances within the
+// thickness; the hypot was most of a sample's work.
+__device__ __forceinline__ double dist_within(const Closest& c, double thickness) {
+  const double r2 = norm2(c);
+  if (thickness >= 1e-100 && thickness <= 1e100 && r2 <= 1e200 && r2 > thickness * thickness * (1 + 1e-9))
+    return __builtin_inf();
+  return jsm::hypot3(c.rx, c.ry, c.rz);
+}
+
+constexpr int kCcdSamples = 16;
+
+// The sampled fallback's answer from each lane's first smallest sample
+// (distance, index): kLanes neighbouring lanes hold one stencil and took every
+// kLanes-th sample each.
+template <int kLanes>
+__device__ __forceinline__ double ccd_sampled(double minD, int minK, double thickness) {
+#pragma unroll
+  for (int off = 1; off < kLanes; off *= 2) {
+    const double d = __shfl_xor(minD, off, kWave);
+    const int k = __shfl_xor(minK, off, kWave);
+    if (d < minD || (d == minD && k < minK)) {
+      minD = d;
+      minK = k;
+    }
+  }
+  return minD <= thickness ? (double)minK / kCcdSamples : __builtin_inf();
+}
+
+// vtCCD() ccd-vt.ts:20-115 after its head (ccd_head); slots 0..3 = p, a, b,
+// c.  kLanes > 1: neighbouring lanes share the stencil, lane `sub` of them.
+template <int kLanes>
+__device__ inline double vt_ccd_tail(const Seg4& S, double thickness, int sub) {
   double p0[3], dp[3], a0[3], da[3], b0[3], db[3], c0[3], dc[3];
   for (int i = 0; i < 3; i++) {
     p0[i] = S.x0[0][i]; dp[i] = S.x1[0][i] - S.x0[0][i];
@@ -324,24 +353,24 @@ __device__ inline double vt_ccd(const Seg4& S, double thickness) {
       pp[i] = p0[i] + dp[i] * t; aa[i] = a0[i] + da[i] * t;
       bb[i] = b0[i] + db[i] * t; cc[i] = c0[i] + dc[i] * t;
     }
-    if (closest_vt(pp, aa, bb, cc).dist <= thickness) return t;
+    if (dist_within(closest_vt<false>(pp, aa, bb, cc), thickness) <= thickness) return t;
   }
-  double minD = __builtin_inf(), minT = 0;
-  const int N = 16;
-  for (int k = 0; k <= N; k++) {
-    const double t = (double)k / N;
+  double minD = __builtin_inf();
+  int minK = 0;
+  for (int k = sub; k <= kCcdSamples; k += kLanes) {
+    const double t = (double)k / kCcdSamples;
     double pp[3], aa[3], bb[3], cc[3];
     for (int i = 0; i < 3; i++) {
       pp[i] = p0[i] + dp[i] * t; aa[i] = a0[i] + da[i] * t;
       bb[i] = b0[i] + db[i] * t; cc[i] = c0[i] + dc[i] * t;
     }
-    const double d = closest_vt(pp, aa, bb, cc).dist;
-    if (d < minD) { minD = d; minT = t; }
+    const double d = dist_within(closest_vt<false>(pp, aa, bb, cc), thickness);
+    if (d < minD) { minD = d; minK = k; }
   }
-  if (minD <= thickness) return minT;
-  return __builtin_inf();
+  return ccd_sampled<kLanes>(minD, minK, thickness);
 }
 
+template <bool kDist = true>
 __device__ __forceinline__ Closest ee_at(const double* a0, const double* da, const double* b0, const double* db,
                                          const double* c0, const double* dc, const double* d0, const double* dd,
                                          double t) {
@@ -350,11 +379,12 @@ __device__ __forceinline__ Closest ee_at(const double* a0, const double* da, con
     A[i] = a0[i] + da[i] * t; B[i] = b0[i] + db[i] * t;
     Cc[i] = c0[i] + dc[i] * t; D[i] = d0[i] + dd[i] * t;
   }
-  return closest_ee(A, B, Cc, D);
+  return closest_ee<kDist>(A, B, Cc, D);
 }
 
-// eeCCD() ccd-ee.ts:24-101; slots 0..3 = a, b, c, d.
-__device__ inline double ee_ccd(const Seg4& S, double thickness) {
+// eeCCD() ccd-ee.ts:24-101 after its head; slots 0..3 = a, b, c, d.
+template <int kLanes>
+__device__ inline double ee_ccd_tail(const Seg4& S, double thickness, int sub) {
   double a0[3], da[3], b0[3], db[3], c0[3], dc[3], d0[3], dd[3];
   for (int i = 0; i < 3; i++) {
     a0[i] = S.x0[0][i]; da[i] = S.x1[0][i] - S.x0[0][i];
@@ -362,10 +392,6 @@ __device__ inline double ee_ccd(const Seg4& S, double thickness) {
     c0[i] = S.x0[2][i]; dc[i] = S.x1[2][i] - S.x0[2][i];
     d0[i] = S.x0[3][i]; dd[i] = S.x1[3][i] - S.x0[3][i];
   }
-  const double q0 = ee_at(a0, da, b0, db, c0, dc, d0, dd, 0).dist;
-  if (q0 <= thickness) return 0;
-  const double dev = stencil_dev(S);
-  if (q0 - 4 * dev > thickness) return __builtin_inf();
   double e10[3], de1[3], e20[3], de2[3], r0[3], dr[3];
   for (int i = 0; i < 3; i++) {
     e10[i] = b0[i] - a0[i]; de1[i] = db[i] - da[i];
@@ -385,18 +411,27 @@ __device__ inline double ee_ccd(const Seg4& S, double thickness) {
   const int nr = solve_cubic01(c3c, c2c, c1c, c0c, roots);
   for (int k = 0; k < nr; k++) {
     const double t = roots[k];
-    const Closest cp = ee_at(a0, da, b0, db, c0, dc, d0, dd, t);
-    if (cp.dist <= thickness && cp.s >= -1e-6 && cp.s <= 1 + 1e-6 && cp.t >= -1e-6 && cp.t <= 1 + 1e-6) return t;
+    const Closest cp = ee_at<false>(a0, da, b0, db, c0, dc, d0, dd, t);
+    if (dist_within(cp, thickness) <= thickness && cp.s >= -1e-6 && cp.s <= 1 + 1e-6 && cp.t >= -1e-6 && cp.t <= 1 + 1e-6) return t;
   }
-  double minD = __builtin_inf(), minT = 0;
-  const int N = 16;
-  for (int k = 0; k <= N; k++) {
-    const double t = (double)k / N;
-    const double d2 = ee_at(a0, da, b0, db, c0, dc, d0, dd, t).dist;
-    if (d2 < minD) { minD = d2; minT = t; }
+  double minD = __builtin_inf();
+  int minK = 0;
+  for (int k = sub; k <= kCcdSamples; k += kLanes) {
+    const double t = (double)k / kCcdSamples;
+    const double d2 = dist_within(ee_at<false>(a0, da, b0, db, c0, dc, d0, dd, t), thickness);
+    if (d2 < minD) { minD = d2; minK = k; }
   }
-  if (minD <= thickness) return minT;
-  return __builtin_inf();
+  return ccd_sampled<kLanes>(minD, minK, thickness);
+}
+
+// vtCCD / eeCCD whole, one lane.
+__device__ inline double vt_ccd(const Seg4& S, double thickness) {
+  double toi;
+  return ccd_head(S, 0, thickness, toi) ? toi : vt_ccd_tail<1>(S, thickness, 0);
+}
+__device__ inline double ee_ccd(const Seg4& S, double thickness) {
+  double toi;
+  return ccd_head(S, 1, thickness, toi) ? toi : ee_ccd_tail<1>(S, thickness, 0);
 }
 
 // barrier.ts:4-24

@@ -48,7 +48,7 @@ struct CScalars {
   unsigned tickets[16];
   uint64_t mink[16];   // okey images of LtMin reductions (all ones = no value)
   uint32_t pair_count, spair_count, active_count, entry_count, nonfinite, floor_fail, nverts, kill_rounds;
-  uint32_t tail_count;
+  uint32_t tail_count[2];  // vertex/triangle, edge/edge
   uint32_t kind_count[4];
   uint32_t todo_count;
   uint64_t nan_key, cross_key;
@@ -2114,7 +2114,8 @@ __global__ void __launch_bounds__(kBlock) k_trial_prims(DGeom G, const double* _
                                                         const double* __restrict__ xt,
                                                         const uint2* __restrict__ pairs, uint32_t np,
                                                         const uint2* __restrict__ spairs,
-                                                        const uint32_t* __restrict__ todo, uint2* tail, CScalars* cs) {
+                                                        const uint32_t* __restrict__ todo, uint2* tail, size_t tail_cap,
+                                                        CScalars* cs) {
   const uint32_t cnt = cs->todo_count, items = (cnt + kWave - 1) / kWave * kTrialParts;
   double minD = __builtin_inf(), minT = __builtin_inf();
   constexpr uint32_t kWaves = kBlock / kWave;
@@ -2159,8 +2160,12 @@ __global__ void __launch_bounds__(kBlock) k_trial_prims(DGeom G, const double* _
           }
         }
       }
-      const uint32_t slot = wave_alloc(queue, &cs->tail_count);
-      if (queue) tail[slot] = make_uint2(j, (uint32_t)k);
+      // vertex/triangle items from the front of the queue, edge/edge from the
+      // back (a static pair's edges begin at k = 3)
+      const bool is_ee = k >= (stat ? 3 : 6);
+      const uint32_t vs = wave_alloc(queue && !is_ee, &cs->tail_count[0]);
+      const uint32_t es = wave_alloc(queue && is_ee, &cs->tail_count[1]);
+      if (queue) tail[is_ee ? tail_cap - 1 - es : vs] = make_uint2(j, (uint32_t)k);
     }
   }
   block_min_to(minD, &cs->mink[5]);
@@ -2168,16 +2173,26 @@ __global__ void __launch_bounds__(kBlock) k_trial_prims(DGeom G, const double* _
 }
 
 // The CCD tail (cubic roots, sampled fallback) of the prims k_trial_prims
-// queued; the queue length is read on the device.
+// queued; the queue lengths are read on the device.  Bound by the chain of one
+// item: kTailLanes lanes share its samples, and a wave has vertex/triangle
+// items (the front of the queue) or edge/edge ones (its back) only.
+constexpr int kTailLanes = 4;
 __global__ void __launch_bounds__(kBlock) k_trial_ccd(DGeom G, const double* __restrict__ xs,
                                                       const double* __restrict__ xt,
                                                       const uint2* __restrict__ pairs, uint32_t np,
                                                       const uint2* __restrict__ spairs,
-                                                      const uint2* __restrict__ tail, CScalars* cs) {
-  const uint32_t cnt = cs->tail_count;
+                                                      const uint2* __restrict__ tail, size_t tail_cap, CScalars* cs) {
+  constexpr uint32_t kPer = kWave / kTailLanes;
+  const uint32_t vt = cs->tail_count[0], ee = cs->tail_count[1];
+  const uint32_t vw = (vt + kPer - 1) / kPer, ew = (ee + kPer - 1) / kPer;
+  const uint32_t lane = threadIdx.x % kWave;
+  const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) / kWave));
   double minT = __builtin_inf();
-  for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < cnt; j += gridDim.x * blockDim.x) {
-    const uint2 it = tail[j];
+  for (uint32_t w = first; w < vw + ew; w += gridDim.x * (kBlock / kWave)) {
+    const bool is_ee = w >= vw;
+    const uint32_t j = (is_ee ? w - vw : w) * kPer + lane / kTailLanes;
+    if (j >= (is_ee ? ee : vt)) continue;
+    const uint2 it = tail[is_ee ? tail_cap - 1 - j : j];
     const bool stat = it.x >= np;
     const uint2 pr = stat ? spairs[it.x - np] : pairs[it.x];
     PairCorners P;
@@ -2194,8 +2209,9 @@ __global__ void __launch_bounds__(kBlock) k_trial_ccd(DGeom G, const double* __r
       vpos(G, xs, ids[s], S.x0[s]);
       vpos(G, xt, ids[s], S.x1[s]);
     }
-    const double toi = q.kind == 0 ? vt_ccd(S, G.d_min) : ee_ccd(S, G.d_min);
-    trial_toi(G, q, toi, minT, cs);
+    const int sub = (int)(lane % kTailLanes);
+    const double toi = is_ee ? ee_ccd_tail<kTailLanes>(S, G.d_min, sub) : vt_ccd_tail<kTailLanes>(S, G.d_min, sub);
+    if (sub == 0) trial_toi(G, q, toi, minT, cs);
   }
   block_min_to(minT, &cs->mink[6]);
 }
@@ -3044,10 +3060,10 @@ struct ContactImpl {
       tune_trial.after_launch(st);
       const dim3 pg(std::min(grid_for((size_t)total * kTrialParts), 2048u));
       hipLaunchKernelGGL(k_trial_prims, pg, dim3(kBlock), 0, st, G, xstep, xt, src.p, src.np, src.s, todo.ptr,
-                         tailq.ptr, cs.ptr);
+                         tailq.ptr, tail_cap, cs.ptr);
       const dim3 cg(tune_ccd.grid((size_t)1 << 40, st));
       hipLaunchKernelGGL(k_trial_ccd, cg, dim3(kBlock), 0, st, G, xstep, xt, src.p, src.np, src.s, tailq.ptr,
-                         cs.ptr);
+                         tail_cap, cs.ptr);
       tune_ccd.after_launch(st);
     }
     if (has_floor)
