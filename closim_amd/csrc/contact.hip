@@ -2372,6 +2372,7 @@ struct ContactImpl {
   DevBuf<uint32_t> kcnt, klist;    // counters / frontier lists of the global-memory sweep
   size_t kill_lds_max = 0;         // dynamic LDS the LDS sweep may use
   size_t flow_lds_max = 0;         // and the dataflow sweep
+  bool repeated_corner = false;    // some triangle names a vertex twice
   DevBuf<double> cg, fr, coeff, dd, hvsum, hterm;
   DevBuf<uint32_t> heads, cverts;
   // lagged friction table
@@ -2460,6 +2461,10 @@ struct ContactImpl {
     for (size_t k = 0; k < (size_t)ms * 3; k++)
       if (d.static_idx[k] >= ns) throw std::invalid_argument("static triangle index out of range");
     idx.upload(d.indices, (size_t)m * 3, st);
+    for (size_t t = 0; t < m; t++) {
+      const uint32_t a = d.indices[t * 3], b = d.indices[t * 3 + 1], c = d.indices[t * 3 + 2];
+      repeated_corner = repeated_corner || a == b || b == c || c == a;
+    }
     if (ms) {
       h_sidx.assign(d.static_idx, d.static_idx + (size_t)ms * 3);
       sidx.upload(d.static_idx, (size_t)ms * 3, st);
@@ -2981,7 +2986,12 @@ struct ContactImpl {
     if (!C) return;
     // heads[] (n entries) serves as the vertex -> LDS slot map here
     hipLaunchKernelGGL(k_kill_slots, dim3(grid_for(nv)), dim3(kBlock), 0, st, cverts.ptr, nv, heads.ptr);
-    if (nv <= kFlowMaxSlot && C <= kFlowMaxRank && flow_lds_bytes(nv) <= flow_lds_max) {
+    // The dataflow sweep runs a contact when each of its vertices has run
+    // exactly `rank` contacts, so a contact must not have two ranks on one
+    // vertex: it would wait for itself.  Pairs that share a vertex are no
+    // candidates, which leaves triangles that name a vertex twice; the
+    // round-based sweep ends on those too (it leaves such contacts out).
+    if (!repeated_corner && nv <= kFlowMaxSlot && C <= kFlowMaxRank && flow_lds_bytes(nv) <= flow_lds_max) {
       ensure_sort(C);
       hipLaunchKernelGGL(k_flow_owner, dim3(grid_for(C)), dim3(kBlock), 0, st, act.ptr, C, akeys.ptr, avals.ptr);
       const bool in_tmp = radix_sort_pairs(st, akeys.ptr, avals.ptr, akeys_t.ptr, avals_t.ptr, C, 0, 8, sort);

@@ -2,8 +2,8 @@
 where its sweep changes hands: fewer contact vertices than the dataflow
 sweep's 64 lanes, exactly as many, a few more, several layers (edge pairs and
 triangles that wait for each other), static partners (contacts with missing
-cloth vertices) and more contact vertices than fit its LDS (the round-based
-sweep).  FP64 steps against the oracle, bit for bit: the sweep performs the
+cloth vertices), more contact vertices than fit its LDS (the round-based
+sweep) and triangles that name a vertex twice (which only that one takes).  FP64 steps against the oracle, bit for bit: the sweep performs the
 reference's operations in list order per vertex, so the bound is equality."""
 import numpy as np
 import pytest
@@ -53,3 +53,67 @@ def test_filter_matches_oracle(nx, ny, count):
 @pytest.mark.parametrize("name", ["plate", "crumpled"])
 def test_filter_with_static_partners_and_folds(name):
     assert check(ALL[name])["active_pairs"] > 0
+
+
+def with_repeated_corner(scene):
+    """The scene with one more triangle, weightless, that names a vertex twice."""
+    me = scene.mesh
+    v, w = me.count - 10, me.count - 3
+    me.indices = np.concatenate([me.indices, np.array([v, w, v], np.uint32)])
+    me.inv_dm = np.concatenate([me.inv_dm, np.zeros(4, np.float32)])
+    me.areas = np.concatenate([me.areas, np.zeros(1, np.float32)])
+    me.tri_count += 1
+    return scene
+
+
+def sweep_without_stuck(ids, vals, v):
+    """killApproachVelocity in list order, without the contacts that name a
+    vertex twice and all that wait for them: what a sweep does that runs a
+    contact once the earlier ones on its vertices have run."""
+    stuck, left = set(), 0
+    for (kind, p, a, b, c, d), val in zip(ids.tolist(), vals):
+        w, nrm = val[:4], val[4:]
+        vs = [p] if kind == 2 else [p, a, b, c] if kind == 0 else [a, b, c, d]
+        if len(set(vs)) < len(vs) or stuck & set(vs):
+            stuck |= set(vs)
+            left += 1
+            continue
+        if kind == 2:
+            v[p, 1] = max(v[p, 1], 0.0)
+        elif kind == 0:
+            t = w[0] * v[a] + w[1] * v[b] + w[2] * v[c]
+            r = v[p] - t
+            rel = r[0] * nrm[0] + r[1] * nrm[1] + r[2] * nrm[2]
+            if rel < 0:
+                j = -0.5 * rel
+                v[p] += j * nrm
+                for k, q in enumerate((a, b, c)):
+                    v[q] -= j * w[k] * nrm
+        else:
+            r = (v[a] + v[b]) / 2 - (v[c] + v[d]) / 2
+            rel = r[0] * nrm[0] + r[1] * nrm[1] + r[2] * nrm[2]
+            if rel < 0:
+                j = -0.25 * rel
+                for q in (a, b):
+                    v[q] += j * nrm
+                for q in (c, d):
+                    v[q] -= j * nrm
+    return left
+
+
+def test_triangle_that_names_a_vertex_twice():
+    # the step ends, and every contact that waits for no such contact has run
+    sc = with_repeated_corner(layers(6, 6, 2))
+    x0 = sc.positions.copy()
+    g = HipSolver("fp64", newton_iters=1, pcg_max_iters=5)
+    g.initialize(sc)
+    g.step(1 / 60)
+    x1, v1 = g.getPositions().copy(), g.getVelocities().copy()
+    assert np.isfinite(x1).all() and np.isfinite(v1).all()
+    ids, vals, _ = g.probe_active_set(x0, x1)
+    damp = 1 - min(max(DEFAULT_MATERIAL.damping, 0), 0.1)
+    v = ((x1 - x0) / (1 / 60) * damp).reshape(-1, 3)
+    left = sweep_without_stuck(ids, vals, v)
+    print(f"{len(ids)} contacts, {left} left out", flush=True)
+    assert 0 < left < len(ids)
+    assert np.max(np.abs(v.reshape(-1) - v1)) <= 1e-12 * np.max(np.abs(v1))
