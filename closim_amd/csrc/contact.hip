@@ -1971,6 +1971,9 @@ __global__ void __launch_bounds__(kFlowWaves * kWave) k_kill_flow(const KillFlow
     bool have = false, have_nxt = false;
     KillFlowRec c = {}, nxt = {};
     while (__ballot(have || have_nxt || taken < cnt)) {
+      // what other lanes wrote in the passes before is read anew (an order
+      // for the compiler: the wave's LDS accesses are in order anyway)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
       FlowVert q[4];
 #pragma unroll
       for (int s = 0; s < 4; s++) {
