@@ -57,6 +57,8 @@ class ContactSystem {
   void friction_xstep_adjoint(const double* x, const double* lam, double* out);
   void commit(const double* x);                            // commit :475-485
   void kill_approach_velocity(const double* x, double* v); // newton.ts:238-303
+  // bound on the dataflow sweep's passes; has it given up?
+  bool filter_wait(uint32_t passes);
   cs_contact_diag diagnostics() const;
   DContactHvp hvp_hook();
   uint64_t active_count() const;

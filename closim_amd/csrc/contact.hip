@@ -1764,13 +1764,19 @@ __global__ void __launch_bounds__(kKillBlock) k_kill_run(const KillRec* __restri
 // one contact; waves 1..4 keep each lane's next records in an LDS ring (wave w
 // the w-th 16 bytes of a record), so no pass waits for memory.
 // Measured (kernel): two 33x33 sheets, 139,462 contacts, depth 15,802: 79.9 ms
-// with k_kill_run<false>, 16.2 ms here; the 256x256 drape on its sphere, 5,164
-// contacts, depth 1,702: 2.35 ms with the LDS form of k_kill_run, 1.35 ms here.
+// with k_kill_run<false>, 16.4 ms here; the 256x256 drape on its sphere, 5,164
+// contacts, depth 1,702: 2.35 ms with the LDS form of k_kill_run, 1.37 ms here
+// (16.15 and 1.36 ms without a bound on the passes).
 
 constexpr uint32_t kFlowLanes = 64, kFlowRing = 8, kFlowBatch = 4;
 constexpr int kFlowWaves = 5;                    // the consumer and four producers
 constexpr uint32_t kFlowMaxRank = (1u << 18) - 1;
 constexpr uint32_t kFlowMaxSlot = (1u << 12) - 1;
+constexpr uint32_t kFlowGaveUp = 0xffffffffu;    // as the number of rounds
+// Passes after which the sweep gives up.  A pass runs at least one contact or
+// waits for memory; 139,462 contacts took 21,000 passes, so this many mean that
+// it would not end (under five seconds at the largest count).
+static uint32_t flow_pass_bound(uint32_t C) { return (1u << 20) + 64 * C; }
 
 // 64 bytes: four 16-byte chunks.  meta[s]: LDS slot of vertex s (bits 0-11),
 // bit 12 set when there is none (static, or a floor contact's unused slots),
@@ -1923,32 +1929,34 @@ __device__ __forceinline__ uint32_t flow_lower(const uint64_t* __restrict__ key,
 __global__ void __launch_bounds__(kFlowWaves * kWave) k_kill_flow(const KillFlowRec* __restrict__ rec,
                                                                   const uint64_t* __restrict__ key, uint32_t C,
                                                                   const uint32_t* __restrict__ cverts, uint32_t nv,
-                                                                  double* v, uint32_t* rounds_out) {
+                                                                  double* v, uint32_t pass_max, uint32_t* rounds_out) {
   extern __shared__ __align__(16) unsigned char flow_lds[];
   double2* Vxy = reinterpret_cast<double2*>(flow_lds);         // [nv] x, y
   FlowZ* Vz = reinterpret_cast<FlowZ*>(Vxy + nv);              // [nv] z, done, level
   uint4* ring = reinterpret_cast<uint4*>(Vz + nv);             // [kFlowRing][4][kFlowLanes]
   uint32_t* tails = reinterpret_cast<uint32_t*>(ring + kFlowRing * 4 * kFlowLanes);  // [kFlowLanes][4]: records in the ring
   uint32_t* heads = tails + 4 * kFlowLanes;                    // [kFlowLanes]: records taken out
+  uint32_t* gave_up = heads + kFlowLanes;                      // [1]
   const uint32_t lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
   for (uint32_t k = threadIdx.x; k < nv; k += blockDim.x) {
     const size_t u = cverts[k];
     Vxy[k] = make_double2(v[u * 3], v[u * 3 + 1]);
     Vz[k] = FlowZ{v[u * 3 + 2], 0, 0};
   }
-  for (uint32_t k = threadIdx.x; k < 5 * kFlowLanes; k += blockDim.x) tails[k] = 0;  // heads follow
+  for (uint32_t k = threadIdx.x; k < 5 * kFlowLanes + 1; k += blockDim.x) tails[k] = 0;  // heads, gave_up follow
   const uint32_t beg = flow_lower(key, C, lane), cnt = flow_lower(key, C, lane + 1) - beg;
   __syncthreads();
   if (wid) {
     // producers: each pass moves up to kFlowBatch records of every lane, and
-    // the loop ends when all records of the wave's lanes are in the ring
-    // (the consumer never stops taking them out)
+    // the loop ends when all records of the wave's lanes are in the ring (the
+    // consumer takes them out until it gives up)
     const uint4* src = reinterpret_cast<const uint4*>(rec) + (wid - 1);
     uint32_t tail = 0;
     while (__ballot(tail < cnt)) {
       const uint32_t head = __hip_atomic_load(&heads[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       const uint32_t nb = min(min(cnt - tail, head + kFlowRing - tail), kFlowBatch);
       if (!__ballot(nb != 0)) {
+        if (__hip_atomic_load(gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) break;
         __builtin_amdgcn_s_sleep(1);
         continue;
       }
@@ -1970,7 +1978,9 @@ __global__ void __launch_bounds__(kFlowWaves * kWave) k_kill_flow(const KillFlow
     uint32_t taken = 0, avail = 0, top = 0;  // records taken from the ring, known to be in it, longest chain
     bool have = false, have_nxt = false;
     KillFlowRec c = {}, nxt = {};
-    while (__ballot(have || have_nxt || taken < cnt)) {
+    // (one branch for both conditions: with two the sweeps took 3 to 4 % longer)
+    uint64_t more;  // lanes with contacts left
+    for (uint32_t pass = pass_max; (more = __ballot(have || have_nxt || taken < cnt)) & (pass ? ~0ull : 0ull); pass--) {
       // what other lanes wrote in the passes before is read anew (an order
       // for the compiler: the wave's LDS accesses are in order anyway)
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
@@ -2041,10 +2051,15 @@ __global__ void __launch_bounds__(kFlowWaves * kWave) k_kill_flow(const KillFlow
         __hip_atomic_store(&heads[lane], taken, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
     }
+    if (more && lane == 0) __hip_atomic_store(gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     for (int off = kWave / 2; off > 0; off >>= 1) top = max(top, (uint32_t)__shfl_down((int)top, off, kWave));
     if (lane == 0) *rounds_out = top;
   }
   __syncthreads();
+  if (*gave_up) {
+    if (threadIdx.x == 0) *rounds_out = kFlowGaveUp;  // (after the same thread's store above)
+    return;
+  }
   for (uint32_t k = threadIdx.x; k < nv; k += blockDim.x) {
     const size_t u = cverts[k];
     v[u * 3] = Vxy[k].x;
@@ -2054,7 +2069,8 @@ __global__ void __launch_bounds__(kFlowWaves * kWave) k_kill_flow(const KillFlow
 }
 
 static size_t flow_lds_bytes(uint32_t nv) {
-  return (size_t)nv * (sizeof(double2) + sizeof(FlowZ)) + (size_t)kFlowRing * 4 * kFlowLanes * sizeof(uint4) + 5 * kFlowLanes * 4;
+  return (size_t)nv * (sizeof(double2) + sizeof(FlowZ)) + (size_t)kFlowRing * 4 * kFlowLanes * sizeof(uint4) +
+         (5 * kFlowLanes + 1) * sizeof(uint32_t);
 }
 
 // checkTrial prims (contact-assembly.ts:497-535) per pair; pairs [0, np)
@@ -2376,6 +2392,8 @@ struct ContactImpl {
   size_t kill_lds_max = 0;         // dynamic LDS the LDS sweep may use
   size_t flow_lds_max = 0;         // and the dataflow sweep
   bool repeated_corner = false;    // some triangle names a vertex twice
+  bool flow_off = false;           // the dataflow sweep gave up once
+  uint32_t flow_pass_max = UINT32_MAX;  // flow_pass_bound unless less
   DevBuf<double> cg, fr, coeff, dd, hvsum, hterm;
   DevBuf<uint32_t> heads, cverts;
   // lagged friction table
@@ -2994,7 +3012,7 @@ struct ContactImpl {
     // vertex: it would wait for itself.  Pairs that share a vertex are no
     // candidates, which leaves triangles that name a vertex twice; the
     // round-based sweep ends on those too (it leaves such contacts out).
-    if (!repeated_corner && nv <= kFlowMaxSlot && C <= kFlowMaxRank && flow_lds_bytes(nv) <= flow_lds_max) {
+    if (!repeated_corner && !flow_off && nv <= kFlowMaxSlot && C <= kFlowMaxRank && flow_lds_bytes(nv) <= flow_lds_max) {
       ensure_sort(C);
       hipLaunchKernelGGL(k_flow_owner, dim3(grid_for(C)), dim3(kBlock), 0, st, act.ptr, C, akeys.ptr, avals.ptr);
       const bool in_tmp = radix_sort_pairs(st, akeys.ptr, avals.ptr, akeys_t.ptr, avals_t.ptr, C, 0, 8, sort);
@@ -3004,11 +3022,16 @@ struct ContactImpl {
       hipLaunchKernelGGL(k_flow_rank, dim3(grid_for(E)), dim3(kBlock), 0, st, v_off.ptr, v_ent.ptr, ent_vtx.ptr, E,
                          kcnt.ptr, kflow.ptr);
       hipLaunchKernelGGL(k_kill_flow, dim3(1), dim3(kFlowWaves * kWave), flow_lds_bytes(nv), st, kflow.ptr,
-                         in_tmp ? akeys_t.ptr : akeys.ptr, C, cverts.ptr, nv, v, &cs.ptr->kill_rounds);
+                         in_tmp ? akeys_t.ptr : akeys.ptr, C, cverts.ptr, nv, v,
+                         std::min(flow_pass_max, flow_pass_bound(C)),
+                         &cs.ptr->kill_rounds);
       CS_LAUNCH_CHECK();
       sync_cs();
-      diag.filter_rounds = hcs->kill_rounds;
-      return;
+      if (hcs->kill_rounds != kFlowGaveUp) {
+        diag.filter_rounds = hcs->kill_rounds;
+        return;
+      }
+      flow_off = true;  // the velocities are as they were: the round-based sweep takes over
     }
     hipLaunchKernelGGL(k_kill_rec, dim3(grid_for(C)), dim3(kBlock), 0, st, act.ptr, C, heads.ptr, krec.ptr);
     hipLaunchKernelGGL(k_kill_links, dim3(grid_for(E)), dim3(kBlock), 0, st, v_off.ptr, v_ent.ptr, ent_vtx.ptr, E,
@@ -3204,6 +3227,10 @@ void ContactSystem::friction_xstep_adjoint(const double* x, const double* lam, d
 void ContactSystem::add_rejection() { im_->diag.rejected_line_search_steps++; }
 void ContactSystem::commit(const double* x) { im_->commit(x); }
 void ContactSystem::kill_approach_velocity(const double* x, double* v) { im_->kill_approach_velocity(x, v); }
+bool ContactSystem::filter_wait(uint32_t passes) {
+  im_->flow_pass_max = passes;
+  return im_->flow_off;
+}
 cs_contact_diag ContactSystem::diagnostics() const {
   im_->settle();
   return im_->diag;

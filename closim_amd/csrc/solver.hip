@@ -1687,6 +1687,14 @@ int cs_hvp_layout(cs_solver* s, uint32_t* tiles) {
   return CS_OK;
 }
 
+int cs_probe_filter_wait(cs_solver* s, uint32_t passes, int32_t* gave_up) {
+  if (!s) return fail(CS_E_NOT_INIT, "CpuSolver not initialized");
+  if (!s->s.contact) return fail(CS_E_INVALID, "solver has no contact system");
+  const bool off = s->s.contact->filter_wait(passes);
+  if (gave_up) *gave_up = off ? 1 : 0;
+  return CS_OK;
+}
+
 int cs_probe_hvp(cs_solver* s, const double* x, const double* p, double inv_h2, double* out) {
   if (!s) return fail(CS_E_NOT_INIT, "CpuSolver not initialized");
   if (!s->s.mixed) return fail(CS_E_INVALID, "solver was not created in mixed precision");

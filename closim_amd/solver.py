@@ -75,6 +75,7 @@ def load_library(path=LIB_PATH):
         "cs_hvp_tiles": (C.c_int, [C.c_void_p, C.POINTER(C.c_uint64), _up, _up, _up, C.POINTER(C.c_uint16),
                                    C.POINTER(C.c_uint16)]),
         "cs_hvp_layout": (C.c_int, [C.c_void_p, C.POINTER(C.c_uint32)]),
+        "cs_probe_filter_wait": (C.c_int, [C.c_void_p, C.c_uint32, C.POINTER(C.c_int32)]),
         "cs_probe_schwarz": (C.c_int, [C.c_void_p, _dp, _dp, _dp, _dp, _dp, C.POINTER(C.c_uint8),
                                        C.POINTER(C.c_uint8), C.POINTER(C.c_uint32)]),
         "cs_probe_active_set": (C.c_int, [C.c_void_p, _dp, _dp, C.POINTER(C.c_int32), _dp, C.c_uint64,
@@ -409,6 +410,14 @@ class HipSolver:
         t = C.c_uint32()
         _check(self._lib.cs_hvp_layout(self._h, C.byref(t)))
         return t.value
+
+    def probe_filter_wait(self, passes):
+        """Bound the dataflow velocity filter's passes; whether it has
+        given up (cs_probe_filter_wait)."""
+        self._need()
+        t = C.c_int32()
+        _check(self._lib.cs_probe_filter_wait(self._h, int(passes), C.byref(t)))
+        return bool(t.value)
 
     def tuned_launch(self):
         """Grid caps the launch autotuner chose for the contact kernels."""

@@ -364,6 +364,12 @@ int cs_hvp_tiles(const cs_scene_desc* scene, uint64_t* sizes, uint32_t* hdr, uin
  * per-vertex gather kernel runs). */
 int cs_hvp_layout(cs_solver* s, uint32_t* tiles);
 
+/* Test hook (no reference counterpart): lowers the number of passes after
+ * which the velocity filter's dataflow sweep ends and leaves its contacts to
+ * the round-based sweep (the same velocities), for the rest of the solver's
+ * life; 0 gives up at once, UINT32_MAX is the default bound.  *gave_up (optional): whether that has happened. */
+int cs_probe_filter_wait(cs_solver* s, uint32_t passes, int32_t* gave_up);
+
 /* Component probe (membraneHvp with the analytic Hessian,
  * membrane-hvp.ts:18-108, plus the inertia term): one launch of the mixed
  * solve's FP32 HVP kernel at (x, p), no contact, pinned rows zeroed:

@@ -117,3 +117,27 @@ def test_triangle_that_names_a_vertex_twice():
     print(f"{len(ids)} contacts, {left} left out", flush=True)
     assert 0 < left < len(ids)
     assert np.max(np.abs(v.reshape(-1) - v1)) <= 1e-12 * np.max(np.abs(v1))
+
+
+@pytest.mark.parametrize("nx,ny,count", [(7, 7, 1), (9, 6, 2)])
+def test_dataflow_sweep_that_gives_up_hands_over(nx, ny, count):
+    # a bound of 0 ends the dataflow sweep before its first contact
+    sg, so = layers(nx, ny, count), layers(nx, ny, count)
+    g = HipSolver("fp64", newton_iters=1, pcg_max_iters=5)
+    g.initialize(sg)
+    o = O.OracleSolver(so, _abi.options(newton_iters=1, pcg_max_iters=5))
+    assert not g.probe_filter_wait(0)
+    for k in range(2):  # the second step does not try again
+        g.step(1 / 60)
+        o.step(1 / 60)
+        assert g.probe_filter_wait(0xFFFFFFFF)
+        assert np.array_equal(g.getPositions(), o.getPositions())
+        assert np.array_equal(g.getVelocities(), o.getVelocities())
+        assert 0 < g.lastStats["contact"]["filter_rounds"] <= g.lastStats["contact"]["active_pairs"]
+
+
+def test_dataflow_sweep_does_not_give_up():
+    g = HipSolver("fp64", newton_iters=1, pcg_max_iters=5)
+    g.initialize(layers(9, 6, 3))
+    g.step(1 / 60)
+    assert not g.probe_filter_wait(0xFFFFFFFF)
