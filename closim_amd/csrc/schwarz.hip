@@ -730,9 +730,11 @@ template <int NC, int ND, int K>
 __global__ void __launch_bounds__(kWave, 1) k_sw_apply64(SwArgs s, const double* __restrict__ r, double* z,
                                                          const int32_t* done) {
   static_assert(kWave % (2 * K) == 0, "blocks come in pairs");
-  // one domain's LDS row: room for the groups read past the end, and a stride
-  // that spreads the domains over the banks
-  constexpr int P = NC * kWave + 18;
+  // One domain's LDS row.  solve_row reads three groups of 8 from the one at
+  // or past the last element on, so up to 24 past the end; that stride also
+  // puts the domains' rows 48 banks apart.
+  constexpr int P = NC * kWave + 24;
+  static_assert((NC * kWave / 8 + 2) * 8 + 8 <= P && P % 2 == 0, "the groups read ahead, and 16-byte loads");
   if (done && *done) return;
   __shared__ __align__(16) double prod[2][ND][P];
   __shared__ double dia[ND][NC * kWave], sub[ND][NC * kWave], ys[ND][NC * kWave];  // L_jj, L_(j+1)j, the forward solution
