@@ -3,9 +3,8 @@
 // of the time.
 #pragma once
 
-#include <atomic>
-
 #include "common.h"
+#include "ticket.h"
 
 namespace cloth {
 
@@ -82,32 +81,20 @@ __device__ __forceinline__ bool coop_exchange(CoopSlots* s, uint32_t& turn, cons
   return false;
 }
 
-// At most kMaxInFlight such launches of this process at once: with 64
-// work-groups of at most 512 threads each they fit the 256 CUs beside each
-// other, so none can keep part of another from becoming resident.  A caller
-// that gets no ticket takes its path of separate kernels (the same results).
-class CoopTicket {
- public:
-  CoopTicket() {
-    int n = count().load();
-    while (n < kMaxInFlight && !count().compare_exchange_weak(n, n + 1)) {
-    }
-    held_ = n < kMaxInFlight;
-  }
-  ~CoopTicket() {
-    if (held_) count().fetch_sub(1);
-  }
-  CoopTicket(const CoopTicket&) = delete;
-  CoopTicket& operator=(const CoopTicket&) = delete;
-  explicit operator bool() const { return held_; }
+static_assert(CoopTicket::kRound == kXcds, "a ticket counts rounds over the XCDs");
 
- private:
-  static constexpr int kMaxInFlight = 4;
-  static std::atomic<int>& count() {
-    static std::atomic<int> n{0};
-    return n;
+// One solver's exchange: its slots, and the compute units it may wait on
+// (those the device has now: a partition or a mask may leave fewer than 256).
+struct CoopState {
+  DevBuf<CoopSlots> slots;
+  int device = -1;
+  unsigned cus = 0;
+  void setup() {  // on the current device
+    CS_HIP(hipGetDevice(&device));
+    int n = 0;
+    CS_HIP(hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device));
+    cus = n > 0 ? (unsigned)n : 0;
   }
-  bool held_ = false;
 };
 
 }  // namespace cloth

@@ -802,7 +802,7 @@ struct MixedImpl {
   DevBuf<float> x32, d32, binv32, sol, r, z, p, Ap, partials, scan;
   DevBuf<Frozen32> act32;
   DevBuf<MxScalars> s;
-  DevBuf<CoopSlots> coop;
+  CoopState coop;
   MxArgs last{};
   bool has_last = false;
 };
@@ -830,6 +830,7 @@ MixedSolve::MixedSolve(const cs_scene_desc& d, const cs_options&, hipStream_t st
   for (auto* b : {&im_->x32, &im_->d32, &im_->sol, &im_->r, &im_->z, &im_->p, &im_->Ap}) b->alloc(n3);
   im_->partials.alloc((size_t)MX_NPART * kMaxRedBlocks);
   im_->s.alloc(1);
+  im_->coop.setup();
   CS_HIP(hipMemsetAsync(im_->s.ptr, 0, sizeof(MxScalars), st));
 }
 
@@ -889,15 +890,16 @@ static int solve_small(MixedImpl& M, const MxArgs& a, const MixedInputs& in) {
   hipStream_t st = M.st;
   const unsigned blocks = mx_hvp_grid(a.me);
   if (!a.me.tl.count || blocks > kCoopMaxBlocks || mx_grid(a.me.n) > blocks) return -1;
-  CoopTicket ticket;
+  CoopTicket ticket(M.coop.device, blocks, M.coop.cus);
   if (!ticket) return -1;
-  M.coop.alloc(1);
-  CS_HIP(hipMemsetAsync(M.coop.ptr, 0xff, sizeof(CoopSlots), st));
-  hipLaunchKernelGGL(k_mx_small, dim3(blocks), dim3(kBlock), 0, st, a, M.coop.ptr, in.max_iters, in.dx);
+  M.coop.slots.alloc(1);
+  CoopSlots* ex = M.coop.slots.ptr;
+  CS_HIP(hipMemsetAsync(ex, 0xff, sizeof(CoopSlots), st));
+  hipLaunchKernelGGL(k_mx_small, dim3(blocks), dim3(kBlock), 0, st, a, ex, in.max_iters, in.dx);
   CS_LAUNCH_CHECK();
   uint64_t gave_up;
   MxScalars hs;
-  CS_HIP(hipMemcpyAsync(&gave_up, &M.coop.ptr->gave_up, sizeof(gave_up), hipMemcpyDeviceToHost, st));
+  CS_HIP(hipMemcpyAsync(&gave_up, &ex->gave_up, sizeof(gave_up), hipMemcpyDeviceToHost, st));
   CS_HIP(hipMemcpyAsync(&hs, M.s.ptr, sizeof(hs), hipMemcpyDeviceToHost, st));
   CS_HIP(hipStreamSynchronize(st));
   if (gave_up != kCoopEmpty) return -1;

@@ -66,10 +66,10 @@ struct PcgArgs {
   Schwarz* sw;         // PRE_SCHWARZ: applied between the kernels (host side only)
 };
 
-// The whole solve in one launch (small meshes); `exchange`: pcg_exchange_bytes()
-// of device memory.  False: not done, solve with the functions below.
-bool pcg_solve_small(hipStream_t st, const PcgArgs& a, int max_iters, void* exchange, PcgScalars* out);
-size_t pcg_exchange_bytes();
+// The whole solve in one launch (small meshes).  False: not done, solve with
+// the functions below.
+struct CoopState;
+bool pcg_solve_small(hipStream_t st, const PcgArgs& a, int max_iters, CoopState& coop, PcgScalars* out);
 void pcg_init(hipStream_t st, const PcgArgs& a);
 // One PCG iteration k (0-based): HVP, then update + preconditioner +
 // residual test + direction update.

@@ -849,13 +849,14 @@ void pcg_init(hipStream_t st, const PcgArgs& a) {
 // contacts (a vertex's entries are summed by its 8 lanes; with many,
 // k_vertex_sums gives them a work-group).  False when it was not done (another
 // path solves it, from the same inputs); *out holds the scalars otherwise.
-bool pcg_solve_small(hipStream_t st, const PcgArgs& a, int max_iters, void* exchange, PcgScalars* out) {
+bool pcg_solve_small(hipStream_t st, const PcgArgs& a, int max_iters, CoopState& coop, PcgScalars* out) {
   const unsigned blocks = (a.me.n + kSmallVerts - 1) / kSmallVerts;
   if (a.precond == PRE_SCHWARZ || blocks > kCoopMaxBlocks || blocks < 1) return false;
   if (a.contact.act && a.contact.nv && use_vertex_groups(a.contact.E, a.contact.nv)) return false;
-  CoopTicket ticket;
+  CoopTicket ticket(coop.device, blocks, coop.cus);
   if (!ticket) return false;
-  CoopSlots* ex = static_cast<CoopSlots*>(exchange);
+  coop.slots.alloc(1);
+  CoopSlots* ex = coop.slots.ptr;
   CS_HIP(hipMemsetAsync(ex, 0xff, sizeof(CoopSlots), st));
   hipLaunchKernelGGL(k_pcg_small, dim3(blocks), dim3(kSmallBlock), 0, st, a, ex, max_iters);
   CS_LAUNCH_CHECK();
@@ -865,7 +866,6 @@ bool pcg_solve_small(hipStream_t st, const PcgArgs& a, int max_iters, void* exch
   CS_HIP(hipStreamSynchronize(st));
   return gave_up == kCoopEmpty;
 }
-size_t pcg_exchange_bytes() { return sizeof(CoopSlots); }
 
 // Back-to-back HVP launches on the operands of the last solve (Ap and the
 // p.Ap partials are overwritten; the latch is cleared for the run and set after).

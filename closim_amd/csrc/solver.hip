@@ -19,6 +19,7 @@
 
 #include "../../include/cloth_hip.h"
 #include "contact.h"
+#include "coop.h"
 #include "fem.h"
 #include "mixed.h"
 #include "pcg.h"
@@ -581,6 +582,7 @@ struct Solver {
       if (id >= n) throw std::invalid_argument("pin id out of range");
     pinmask.alloc(n);
     if (opt.precond == CS_PRECOND_BLOCK_JACOBI) binv.alloc((size_t)n * 9);
+    coop.setup();
     has_contact = d->contact_enabled != 0;
     if (has_contact) contact.reset(new ContactSystem(*d, st));
     if (opt.precision == CS_PREC_MIXED) mixed.reset(new MixedSolve(*d, opt, st));
@@ -1156,7 +1158,7 @@ struct Solver {
     return in;
   }
 
-  DevBuf<uint8_t> pcg_exchange;
+  CoopState coop;
   PcgArgs last_pcg{};
   bool has_last_pcg = false;
 
@@ -1213,9 +1215,8 @@ struct Solver {
     }
     if (!(opt.flags & CS_FLAG_TIMING)) {
       // kernel timing brackets the launches of the separate kernels
-      pcg_exchange.alloc(pcg_exchange_bytes());
       PcgScalars ps;
-      if (pcg_solve_small(st, a, maxIters, pcg_exchange.ptr, &ps)) return k_first_done_zero(ps) ? maxIters : ps.iters;
+      if (pcg_solve_small(st, a, maxIters, coop, &ps)) return k_first_done_zero(ps) ? maxIters : ps.iters;
     }
     pcg_init(st, a);
     const int chunk = 8;

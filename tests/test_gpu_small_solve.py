@@ -11,7 +11,7 @@ import pytest
 import oracle_ffi as O
 from closim_amd import _abi, mesh as M, scenes as S
 from closim_amd.scene import DEFAULT_MATERIAL, create_scene
-from closim_amd.solver import HipSolver
+from closim_amd.solver import HipBatch, HipSolver
 from contact_scenes import ALL
 
 pytestmark = pytest.mark.gpu
@@ -109,3 +109,25 @@ def test_gradient_on_both_sides_of_its_rule(nx, ny):
     o = O.OracleSolver(make(), _abi.options(newton_iters=1, pcg_max_iters=1))
     o.step(H)
     assert np.array_equal(x, o.getPositions()) and np.array_equal(v, o.getVelocities())
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_more_solves_at_once_than_tickets(precision):
+    # six meshes of 64 work-groups each, four of which fit 256 compute units:
+    # whoever gets no ticket takes the separate kernels, with the same results
+    nx, ny = (62, 64) if precision == "fp64" else (110, 139)
+    kw = dict(newton_iters=3)
+    alone = HipSolver(precision, **kw)
+    alone.initialize(hung(nx, ny))
+    gs = [HipSolver(precision, **kw) for _ in range(6)]
+    for g in gs:
+        g.initialize(hung(nx, ny))
+    B = HipBatch(gs, threads=6)
+    for _ in range(2):
+        alone.step(H)
+        assert B.step(H) == [0] * 6
+        for g in gs:
+            assert np.array_equal(g.getPositions(), alone.getPositions())
+            assert np.array_equal(g.getVelocities(), alone.getVelocities())
+    for g in gs:
+        g.close()
