@@ -28,6 +28,10 @@ struct CoopSlots {
   uint64_t w[kCoopSets][kCoopWords][kCoopMaxBlocks];  // set to all ones before each launch
   uint64_t gave_up;                                   // not all ones: some work-group waited in vain
 };
+struct CoopExchange {
+  CoopSlots* s;
+  uint32_t polls;  // before an exchange gives up
+};
 
 template <class T>
 __device__ __forceinline__ T coop_load(const T* p) {
@@ -52,9 +56,10 @@ __device__ __forceinline__ uint64_t coop_word(double x) {
 // has read (each published its words of the exchange in between).  False when
 // the others do not come.
 template <int NW>
-__device__ __forceinline__ bool coop_exchange(CoopSlots* s, uint32_t& turn, const uint64_t (&mine)[NW],
+__device__ __forceinline__ bool coop_exchange(const CoopExchange& ex, uint32_t& turn, const uint64_t (&mine)[NW],
                                               uint64_t (&got)[NW]) {
   static_assert(NW <= (int)kCoopWords, "slot words");
+  CoopSlots* s = ex.s;
   const uint32_t lane = threadIdx.x % kWave, set = turn % kCoopSets, old = (turn + 2) % kCoopSets;
   turn++;
   coop_drain();  // the words emptied last time are, before these can be seen
@@ -66,7 +71,7 @@ __device__ __forceinline__ bool coop_exchange(CoopSlots* s, uint32_t& turn, cons
   const bool in = lane < gridDim.x;
 #pragma unroll
   for (int k = 0; k < NW; k++) got[k] = in ? kCoopEmpty : 0;
-  for (uint32_t i = 0; i < kCoopSpin; i++) {
+  for (uint32_t i = 0; i < ex.polls; i++) {
     bool wait = false;
     if (in)
 #pragma unroll
@@ -89,6 +94,8 @@ struct CoopState {
   DevBuf<CoopSlots> slots;
   int device = -1;
   unsigned cus = 0;
+  uint32_t polls = kCoopSpin;
+  bool gave_up = false;  // an exchange of this solver waited in vain: no such launches any more
   void setup() {  // on the current device
     CS_HIP(hipGetDevice(&device));
     int n = 0;

@@ -37,6 +37,7 @@ struct MixedInputs {
   bool psd = false;       // stress projected to PSD in the HVP (CS_FLAG_PSD_NEWTON)
 };
 
+struct CoopState;
 struct MixedImpl;
 struct PackedScratch;
 class MixedSolve;
@@ -77,6 +78,7 @@ class MixedSolve {
   // The device latch of the last solve: 0 iteration cap, 1 stopped on
   // non-positive curvature (p.Ap <= 1e-30), 2 converged.
   const int32_t* done_flag() const;
+  CoopState& coop();  // the one-launch solve's exchange
   void set_material(const cs_material&) {}
 
  private:

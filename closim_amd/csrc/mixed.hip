@@ -603,7 +603,7 @@ __device__ __forceinline__ uint64_t mx_word(float a, float b) {
 
 // Sums two floats over the work-groups as block_partial_f and
 // merge_partials_f do over at most 64 partials: every thread gets the totals.
-__device__ __forceinline__ bool mx_sums(CoopSlots* ex, uint32_t& turn, float& a, float& b) {
+__device__ __forceinline__ bool mx_sums(const CoopExchange& ex, uint32_t& turn, float& a, float& b) {
   __shared__ float s_tot[2];
   __shared__ int s_ok;
   coop_drain();  // this thread's part of Ap or z
@@ -633,7 +633,7 @@ __device__ __forceinline__ bool mx_sums(CoopSlots* ex, uint32_t& turn, float& a,
   return s_ok != 0;
 }
 
-__global__ void __launch_bounds__(kBlock) k_mx_small(MxArgs a, CoopSlots* ex, int max_iters, double* dx) {
+__global__ void __launch_bounds__(kBlock) k_mx_small(MxArgs a, CoopExchange ex, int max_iters, double* dx) {
   __shared__ float xs[kTileLoc * 3], ps[kTileLoc * 3], out[kTileTris * 9];
   __shared__ uint8_t pin[kTileLoc];
   constexpr int kTriSlots = (kTileTris + kBlock - 1) / kBlock, kEnt = 8;
@@ -834,6 +834,7 @@ MixedSolve::MixedSolve(const cs_scene_desc& d, const cs_options&, hipStream_t st
   CS_HIP(hipMemsetAsync(im_->s.ptr, 0, sizeof(MxScalars), st));
 }
 
+CoopState& MixedSolve::coop() { return im_->coop; }
 const int32_t* MixedSolve::done_flag() const { return &im_->s.ptr->done; }
 
 MixedSolve::~MixedSolve() {
@@ -890,19 +891,22 @@ static int solve_small(MixedImpl& M, const MxArgs& a, const MixedInputs& in) {
   hipStream_t st = M.st;
   const unsigned blocks = mx_hvp_grid(a.me);
   if (!a.me.tl.count || blocks > kCoopMaxBlocks || mx_grid(a.me.n) > blocks) return -1;
+  if (M.coop.gave_up) return -1;
   CoopTicket ticket(M.coop.device, blocks, M.coop.cus);
   if (!ticket) return -1;
   M.coop.slots.alloc(1);
   CoopSlots* ex = M.coop.slots.ptr;
   CS_HIP(hipMemsetAsync(ex, 0xff, sizeof(CoopSlots), st));
-  hipLaunchKernelGGL(k_mx_small, dim3(blocks), dim3(kBlock), 0, st, a, ex, in.max_iters, in.dx);
+  hipLaunchKernelGGL(k_mx_small, dim3(blocks), dim3(kBlock), 0, st, a, CoopExchange{ex, M.coop.polls},
+                     in.max_iters, in.dx);
   CS_LAUNCH_CHECK();
   uint64_t gave_up;
   MxScalars hs;
   CS_HIP(hipMemcpyAsync(&gave_up, &ex->gave_up, sizeof(gave_up), hipMemcpyDeviceToHost, st));
   CS_HIP(hipMemcpyAsync(&hs, M.s.ptr, sizeof(hs), hipMemcpyDeviceToHost, st));
   CS_HIP(hipStreamSynchronize(st));
-  if (gave_up != kCoopEmpty) return -1;
+  M.coop.gave_up = gave_up != kCoopEmpty;
+  if (M.coop.gave_up) return -1;
   return hs.done ? hs.iters : in.max_iters;
 }
 

@@ -616,7 +616,7 @@ __device__ __forceinline__ void sum2_wave(Sum2 (&v)[NQ]) {
 // barrier; with `publish`, vectors written with coop_store before it may be
 // read with plain loads after it.  False when an exchange gave up.
 template <int NQ>
-__device__ __forceinline__ bool small_sums(CoopSlots* ex, uint32_t& turn, Sum2 (&v)[NQ], double (&tot)[NQ],
+__device__ __forceinline__ bool small_sums(const CoopExchange& ex, uint32_t& turn, Sum2 (&v)[NQ], double (&tot)[NQ],
                                            bool publish) {
   __shared__ Sum2 s_wave[NQ][kSmallWaves];
   __shared__ double s_tot[NQ];
@@ -659,7 +659,7 @@ __device__ __forceinline__ bool small_sums(CoopSlots* ex, uint32_t& turn, Sum2 (
   return s_ok != 0;
 }
 
-__global__ void __launch_bounds__(kSmallBlock) k_pcg_small(PcgArgs a, CoopSlots* ex, int max_iters) {
+__global__ void __launch_bounds__(kSmallBlock) k_pcg_small(PcgArgs a, CoopExchange ex, int max_iters) {
   const int sub = threadIdx.x % kLanesPerVertex;
   const int base = (threadIdx.x % kWave) - sub;
   const uint32_t v = blockIdx.x * kSmallVerts + threadIdx.x / kLanesPerVertex;
@@ -853,18 +853,20 @@ bool pcg_solve_small(hipStream_t st, const PcgArgs& a, int max_iters, CoopState&
   const unsigned blocks = (a.me.n + kSmallVerts - 1) / kSmallVerts;
   if (a.precond == PRE_SCHWARZ || blocks > kCoopMaxBlocks || blocks < 1) return false;
   if (a.contact.act && a.contact.nv && use_vertex_groups(a.contact.E, a.contact.nv)) return false;
+  if (coop.gave_up) return false;
   CoopTicket ticket(coop.device, blocks, coop.cus);
   if (!ticket) return false;
   coop.slots.alloc(1);
   CoopSlots* ex = coop.slots.ptr;
   CS_HIP(hipMemsetAsync(ex, 0xff, sizeof(CoopSlots), st));
-  hipLaunchKernelGGL(k_pcg_small, dim3(blocks), dim3(kSmallBlock), 0, st, a, ex, max_iters);
+  hipLaunchKernelGGL(k_pcg_small, dim3(blocks), dim3(kSmallBlock), 0, st, a, CoopExchange{ex, coop.polls}, max_iters);
   CS_LAUNCH_CHECK();
   uint64_t gave_up;
   CS_HIP(hipMemcpyAsync(&gave_up, &ex->gave_up, sizeof(gave_up), hipMemcpyDeviceToHost, st));
   CS_HIP(hipMemcpyAsync(out, a.s, sizeof(*out), hipMemcpyDeviceToHost, st));
   CS_HIP(hipStreamSynchronize(st));
-  return gave_up == kCoopEmpty;
+  coop.gave_up = gave_up != kCoopEmpty;
+  return !coop.gave_up;
 }
 
 // Back-to-back HVP launches on the operands of the last solve (Ap and the

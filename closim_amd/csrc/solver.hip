@@ -1696,6 +1696,14 @@ int cs_probe_filter_wait(cs_solver* s, uint32_t passes, int32_t* gave_up) {
   return CS_OK;
 }
 
+int cs_probe_exchange_wait(cs_solver* s, uint32_t polls, int32_t* gave_up) {
+  if (!s) return fail(CS_E_NOT_INIT, "CpuSolver not initialized");
+  cloth::CoopState& c = s->s.mixed ? s->s.mixed->coop() : s->s.coop;
+  c.polls = std::min(polls, cloth::kCoopSpin);
+  if (gave_up) *gave_up = c.gave_up ? 1 : 0;
+  return CS_OK;
+}
+
 int cs_probe_hvp(cs_solver* s, const double* x, const double* p, double inv_h2, double* out) {
   if (!s) return fail(CS_E_NOT_INIT, "CpuSolver not initialized");
   if (!s->s.mixed) return fail(CS_E_INVALID, "solver was not created in mixed precision");

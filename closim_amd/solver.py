@@ -76,6 +76,7 @@ def load_library(path=LIB_PATH):
                                    C.POINTER(C.c_uint16)]),
         "cs_hvp_layout": (C.c_int, [C.c_void_p, C.POINTER(C.c_uint32)]),
         "cs_probe_filter_wait": (C.c_int, [C.c_void_p, C.c_uint32, C.POINTER(C.c_int32)]),
+        "cs_probe_exchange_wait": (C.c_int, [C.c_void_p, C.c_uint32, C.POINTER(C.c_int32)]),
         "cs_probe_schwarz": (C.c_int, [C.c_void_p, _dp, _dp, _dp, _dp, _dp, C.POINTER(C.c_uint8),
                                        C.POINTER(C.c_uint8), C.POINTER(C.c_uint32)]),
         "cs_probe_active_set": (C.c_int, [C.c_void_p, _dp, _dp, C.POINTER(C.c_int32), _dp, C.c_uint64,
@@ -417,6 +418,14 @@ class HipSolver:
         self._need()
         t = C.c_int32()
         _check(self._lib.cs_probe_filter_wait(self._h, int(passes), C.byref(t)))
+        return bool(t.value)
+
+    def probe_exchange_wait(self, polls):
+        """Bound the polls of the one-launch inner solve's exchanges; whether
+        one has given up (cs_probe_exchange_wait)."""
+        self._need()
+        t = C.c_int32()
+        _check(self._lib.cs_probe_exchange_wait(self._h, int(polls), C.byref(t)))
         return bool(t.value)
 
     def tuned_launch(self):

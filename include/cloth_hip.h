@@ -369,6 +369,11 @@ int cs_hvp_layout(cs_solver* s, uint32_t* tiles);
  * the round-based sweep (the same velocities), for the rest of the solver's
  * life; 0 gives up at once, UINT32_MAX is the default bound.  *gave_up (optional): whether that has happened. */
 int cs_probe_filter_wait(cs_solver* s, uint32_t passes, int32_t* gave_up);
+/* The same for the inner solves that run in one launch (small meshes): the
+ * polls after which a wait for the other work-groups ends and the separate
+ * kernels solve the system (the same results), for the rest of the solver's
+ * life; 0 gives up at once, UINT32_MAX is the default bound. */
+int cs_probe_exchange_wait(cs_solver* s, uint32_t polls, int32_t* gave_up);
 
 /* Component probe (membraneHvp with the analytic Hessian,
  * membrane-hvp.ts:18-108, plus the inertia term): one launch of the mixed

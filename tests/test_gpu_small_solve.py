@@ -131,3 +131,25 @@ def test_more_solves_at_once_than_tickets(precision):
             assert np.array_equal(g.getVelocities(), alone.getVelocities())
     for g in gs:
         g.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("nx,ny", [(1, 1), (13, 9), (40, 30)])
+def test_solve_that_gives_up_hands_over(precision, nx, ny):
+    # a bound of 0 polls ends the first exchange of every work-group: the
+    # separate kernels solve from the same inputs and no later solve tries again
+    a, b = HipSolver(precision), HipSolver(precision, flags=_abi.CS_FLAG_TIMING)
+    a.initialize(hung(nx, ny))
+    b.initialize(hung(nx, ny))
+    assert not a.probe_exchange_wait(0)
+    for _ in range(2):
+        a.step(H)
+        b.step(H)
+        assert a.probe_exchange_wait(0xFFFFFFFF)
+        assert a.lastStats["pcg_iters"] == b.lastStats["pcg_iters"]
+        assert np.array_equal(a.getPositions(), b.getPositions())
+        assert np.array_equal(a.getVelocities(), b.getVelocities())
+    c = HipSolver(precision)
+    c.initialize(hung(nx, ny))
+    c.step(H)
+    assert not c.probe_exchange_wait(0xFFFFFFFF)
