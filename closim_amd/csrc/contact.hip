@@ -51,6 +51,7 @@ struct CScalars {
   uint32_t tail_count[2];  // vertex/triangle, edge/edge
   uint32_t kind_count[4];
   uint32_t todo_count;
+  uint32_t most_entries;  // of a vertex
   uint64_t nan_key, cross_key;
 };
 
@@ -1090,17 +1091,28 @@ __global__ void __launch_bounds__(kBlock) k_contact_verts(const uint64_t* __rest
   if (head) cverts[k] = u;
 }
 
-__global__ void k_entry_offsets(const uint64_t* __restrict__ keys, int cshift, uint32_t n, uint32_t* v_off,
-                                const CScalars* cs) {
-  const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x, cnt = cs->entry_count;
-  if (u > n) return;
+// A work-group also finds the most entries of a vertex: its vertices overlap
+// the next one's by one, so that every count is the difference of two lanes.
+constexpr uint32_t kOffsetVerts = kBlock - 1;
+__global__ void __launch_bounds__(kBlock) k_entry_offsets(const uint64_t* __restrict__ keys, int cshift, uint32_t n,
+                                                          uint32_t* v_off, CScalars* cs) {
+  __shared__ uint32_t s_lo[kBlock], s_most;
+  const uint32_t u = blockIdx.x * kOffsetVerts + threadIdx.x, cnt = cs->entry_count;
   uint32_t lo = 0, hi = cnt;
   while (lo < hi) {
     const uint32_t mid = lo + (hi - lo) / 2;
     if ((keys[mid] >> cshift) < (uint64_t)u) lo = mid + 1;
     else hi = mid;
   }
-  v_off[u] = lo;
+  if (u <= n) v_off[u] = lo;
+  s_lo[threadIdx.x] = lo;
+  if (threadIdx.x == 0) s_most = 0;
+  __syncthreads();
+  uint32_t most = threadIdx.x < kOffsetVerts ? s_lo[threadIdx.x + 1] - lo : 0;
+  for (int off = kWave / 2; off > 0; off >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, off, kWave));
+  if (threadIdx.x % kWave == 0) atomicMax(&s_most, most);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_most) atomicMax(&cs->most_entries, s_most);
 }
 
 // ---------------------------------------------------------- per contact
@@ -2833,10 +2845,12 @@ struct ContactImpl {
   int cshift = 3;
   uint32_t E = 0;   // vertex -> contact incidence entries
   uint32_t nv = 0;  // vertices with entries
+  uint32_t most = 0;  // entries of the vertex that has the most
   // (kind, entry and vertex counts start at zero: candidate_source cleared them)
   void build_incidence() {
     E = 0;
     nv = 0;  // no contact vertex until the entries are rebuilt below
+    most = 0;
     if (!C) {
       CS_HIP(hipMemsetAsync(v_off.ptr, 0, (size_t)(n + 1) * sizeof(uint32_t), st));
       sync_cs();
@@ -2857,14 +2871,15 @@ struct ContactImpl {
     // these read the entry count on the device, so that one host read serves all
     hipLaunchKernelGGL(k_entry_ent, dim3(grid_for(nent)), dim3(kBlock), 0, st, sk, cshift, v_ent.ptr, ent_vtx.ptr,
                        cs.ptr);
-    hipLaunchKernelGGL(k_entry_offsets, dim3(grid_for((size_t)n + 1)), dim3(kBlock), 0, st, sk, cshift, n, v_off.ptr,
-                       cs.ptr);
+    hipLaunchKernelGGL(k_entry_offsets, dim3(grid_for((size_t)n + 1, kOffsetVerts)), dim3(kBlock), 0, st, sk, cshift, n,
+                       v_off.ptr, cs.ptr);
     hipLaunchKernelGGL(k_contact_verts, dim3(grid_for(nent)), dim3(kBlock), 0, st, sk, cshift, cverts.ptr, cs.ptr);
     CS_HIP(hipMemsetAsync(hvsum.ptr, 0, (size_t)n * 3 * sizeof(double), st));
     CS_LAUNCH_CHECK();
     sync_cs();
     E = hcs->entry_count;
     nv = E ? hcs->nverts : 0;
+    most = E ? hcs->most_entries : 0;
   }
 
   CEval cev() { return CEval{inr.ptr, cg.ptr, fr.ptr, coeff.ptr}; }
@@ -3387,6 +3402,7 @@ DContactHvp ContactSystem::hvp_hook() {
   h.C = im_->C;
   h.E = im_->E;
   h.nv = im_->nv;
+  h.most = im_->most;
   h.ent_vtx = im_->ent_vtx.ptr;
   h.term = im_->hterm.ptr;
   h.dd = im_->dd.ptr;

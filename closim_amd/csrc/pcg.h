@@ -19,6 +19,7 @@ struct DContactHvp {
   uint32_t C = 0;
   uint32_t E = 0;                    // incidence entries (sorted by vertex, then list order)
   uint32_t nv = 0;                   // vertices with incidence entries
+  uint32_t most = 0;                 // entries of the vertex that has the most
   const Frozen* act = nullptr;
   const uint8_t* inr = nullptr;      // 1 when the contact is inside dHat
   const double* coeff = nullptr;     // kappa * max(b''(d), 0), 0 when d >= dHat

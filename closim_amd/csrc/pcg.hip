@@ -845,14 +845,20 @@ void pcg_init(hipStream_t st, const PcgArgs& a) {
 }
 
 // Solves the system in one launch where that is the faster way: up to
-// kCoopMaxBlocks work-groups of 64 vertices, no Schwarz, and vertices with few
-// contacts (a vertex's entries are summed by its 8 lanes; with many,
-// k_vertex_sums gives them a work-group).  False when it was not done (another
-// path solves it, from the same inputs); *out holds the scalars otherwise.
+// kCoopMaxBlocks work-groups of 64 vertices, no Schwarz, and no vertex with
+// many contacts.  A vertex's entries are summed by its 8 lanes, 8 at a time, and
+// every work-group waits for the longest sum: a step's time per iteration
+// grows by 0.26 us an entry of that vertex.  40x40 sheets on a floor with a
+// finer and finer static grid under one vertex, here / with the separate
+// kernels: 46 / 52 us at 53 entries, 100 / 56 at 273, 195 / 68 at 609, 954 / 157
+// at 3,573 (20x20 and 62x62 sheets alike); the lines meet near 85.  False
+// when it was not done (another path solves it, from the same inputs); *out
+// holds the scalars otherwise.
+constexpr uint32_t kSmallMaxEntries = 64;
 bool pcg_solve_small(hipStream_t st, const PcgArgs& a, int max_iters, CoopState& coop, PcgScalars* out) {
   const unsigned blocks = (a.me.n + kSmallVerts - 1) / kSmallVerts;
   if (a.precond == PRE_SCHWARZ || blocks > kCoopMaxBlocks || blocks < 1) return false;
-  if (a.contact.act && a.contact.nv && use_vertex_groups(a.contact.E, a.contact.nv)) return false;
+  if (a.contact.act && a.contact.nv && a.contact.most > kSmallMaxEntries) return false;
   if (coop.gave_up) return false;
   CoopTicket ticket(coop.device, blocks, coop.cus);
   if (!ticket) return false;

@@ -10,7 +10,7 @@ import pytest
 
 import oracle_ffi as O
 from closim_amd import _abi, mesh as M, scenes as S
-from closim_amd.scene import DEFAULT_MATERIAL, create_scene
+from closim_amd.scene import DEFAULT_CONTACT_PARAMS, DEFAULT_MATERIAL, ContactSystem, create_scene
 from closim_amd.solver import HipBatch, HipSolver
 from contact_scenes import ALL
 
@@ -153,3 +153,41 @@ def test_solve_that_gives_up_hands_over(precision, nx, ny):
     c.initialize(hung(nx, ny))
     c.step(H)
     assert not c.probe_exchange_wait(0xFFFFFFFF)
+
+
+def grid_below(nx, fine):
+    """A sheet sinking on the floor, one vertex of it just above a static grid
+    of fine x fine points, 2 mm from its middle to its sides."""
+    pos, uv, idx = S.merge_parts([S.offset_mesh(nx, nx, 0.004 * nx, 0.004 * nx, 0.0, 0.0013, 0.0)])
+    scene = create_scene(M.preprocess(pos, uv, idx, 0.15), DEFAULT_MATERIAL)
+    scene.positions += np.random.default_rng(nx).uniform(-1e-4, 1e-4, scene.positions.shape)
+    scene.velocities.reshape(-1, 3)[:] = [0.01, -0.03, 0.0]
+    X = scene.positions.reshape(-1, 3)
+    p = X[(nx // 2) * (nx + 1) + nx // 2]
+    at = np.linspace(-0.002, 0.002, fine)
+    V = np.array([[p[0] + a, p[1] - 0.001, p[2] + b] for a in at for b in at], np.float32)
+    q = [a * fine + b for a in range(fine - 1) for b in range(fine - 1)]
+    T = [t for k in q for t in ([k, k + 1, k + fine], [k + 1, k + fine + 1, k + fine])]
+    scene.contact = ContactSystem(DEFAULT_CONTACT_PARAMS)
+    scene.contact.setFloor(0.0)
+    scene.contact.setStaticMesh(V.reshape(-1), np.array(T, np.uint32).reshape(-1))
+    return scene
+
+
+@pytest.mark.parametrize("fine,one_launch", [(2, True), (3, False), (6, False)])
+def test_rule_looks_at_the_vertex_with_the_most_contacts(fine, one_launch):
+    # few contacts a vertex on average, but some 50, 270 and 1,900 on one
+    kw = dict(newton_iters=2)
+    check(lambda: grid_below(12, fine), **kw)
+    g = HipSolver("fp64", **kw)
+    sc = grid_below(12, fine)
+    g.initialize(sc)
+    ids, _, _ = g.probe_active_set(sc.positions, sc.positions)
+    v = np.concatenate([ids[ids[:, 0] == 0][:, 1:5].ravel(), ids[ids[:, 0] == 1][:, 2:6].ravel(),
+                        ids[ids[:, 0] == 2][:, 1]])
+    most = np.bincount(v[v >= 0]).max()
+    print(f"most entries of a vertex {most}", flush=True)
+    assert (most <= 64) == one_launch
+    g.probe_exchange_wait(0)  # the one-launch solve, where it is tried, gives up at once
+    g.step(H)
+    assert g.probe_exchange_wait(0xFFFFFFFF) == one_launch
