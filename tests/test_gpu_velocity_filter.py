@@ -141,3 +141,44 @@ def test_dataflow_sweep_does_not_give_up():
     g.initialize(layers(9, 6, 3))
     g.step(1 / 60)
     assert not g.probe_filter_wait(0xFFFFFFFF)
+
+
+def patches_on_floor_sheet(nx, k):
+    """A floor sheet, and above its middle a patch of k x k cells: many
+    contact vertices, and enough pairs that wait for each other."""
+    parts = [S.offset_mesh(nx, nx, 0.004 * nx, 0.004 * nx, 0.0, 0.0013, 0.0),
+             S.offset_mesh(k, k, 0.004 * k, 0.004 * k, 0.004 * (nx // 2) + 0.001, 0.0026, 0.004 * (nx // 2))]
+    pos, uv, idx = S.merge_parts(parts)
+    scene = create_scene(M.preprocess(pos, uv, idx, 0.15), DEFAULT_MATERIAL)
+    rng = np.random.default_rng(nx)
+    scene.positions += rng.uniform(-1e-4, 1e-4, scene.positions.shape)
+    scene.velocities.reshape(-1, 3)[:] = [0.01, -0.03, 0.0]
+    scene.velocities += rng.uniform(-0.02, 0.02, scene.velocities.shape)
+    scene.contact = ContactSystem(DEFAULT_CONTACT_PARAMS)
+    scene.contact.setFloor(0.0)
+    return scene
+
+
+@pytest.mark.parametrize("nx,k,lds", [(66, 5, True), (80, 8, False)])
+def test_round_based_sweep_with_pairs_matches_oracle(nx, k, lds):
+    # above the dataflow sweep's vertices, in LDS and beyond it: the contacts of
+    # the sweep are the active set at the step's end
+    sg, so = patches_on_floor_sheet(nx, k), patches_on_floor_sheet(nx, k)
+    x0 = sg.positions.copy()
+    g = HipSolver("fp64", newton_iters=1, pcg_max_iters=5)
+    g.initialize(sg)
+    o = O.OracleSolver(so, _abi.options(newton_iters=1, pcg_max_iters=5))
+    g.step(1 / 60)
+    o.step(1 / 60)
+    x1, v1 = g.getPositions().copy(), g.getVelocities().copy()
+    assert np.array_equal(x1, o.getPositions()) and np.array_equal(v1, o.getVelocities())
+    rounds = g.lastStats["contact"]["filter_rounds"]
+    ids, _, _ = g.probe_active_set(x0, x1)
+    v = np.concatenate([ids[ids[:, 0] == 0][:, 1:5].ravel(), ids[ids[:, 0] == 1][:, 2:6].ravel(),
+                        ids[ids[:, 0] == 2][:, 1]])
+    nv, pairs = len(np.unique(v[v >= 0])), int((ids[:, 0] != 2).sum())
+    need = nv * 32 + (len(ids) + 3) // 4 * 4  # velocities, lists and counters of the LDS form
+    print(f"{nv} contact vertices, {len(ids)} contacts, {pairs} pairs, {rounds} rounds, {need} bytes", flush=True)
+    assert nv > 4200  # beyond the dataflow sweep
+    assert (need <= 160 * 1024 - 256) == lds and abs(need - 160 * 1024) > 4096
+    assert pairs > 1000 and rounds > 1
