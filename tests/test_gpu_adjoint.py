@@ -197,3 +197,73 @@ def test_material_adjoint_at_128x128_first_steps_match_fd():
               flush=True)
         assert rel_err(grad[j], fd[j]) < REL, A.PARAMS[j]
     g.close()
+
+
+def compressed(nx, f):
+    """The corner-pinned sheet (a step that came from there) squeezed to f in
+    its plane: its Hessian is indefinite out of the plane."""
+    sc, g = make(nx)
+    P = sc.positions.reshape(-1, 3).copy()
+    P[:, 0] *= f
+    P[:, 2] *= f
+    return g, P.reshape(-1), np.random.default_rng(nx).standard_normal(P.size)
+
+
+def test_adjoint_solve_stops_at_once_where_the_hessian_is_not_positive():
+    # the first direction already has p.Ap <= 0: lambda = 0, so what is left of
+    # the adjoint are the terms without lambda
+    g, x1, w = compressed(8, 0.5)
+    wx = np.zeros_like(w)
+    wx[1::3] = w[1::3]  # out of the plane
+    wv = np.random.default_rng(1).standard_normal(w.size)
+    dx, dv, dth, it, rr = g.step_adjoint(H, x1, np.zeros_like(x1), x1, wx, 1e-3 * wv)
+    damp = 1 - min(max(STRIP_MATERIAL.damping, 0), 0.1)
+    assert it == 0 and rr == 1.0
+    assert np.array_equal(dv, np.zeros_like(dv)) and np.array_equal(dth, np.zeros(5))
+    assert np.allclose(dx, -(damp / H) * 1e-3 * wv, rtol=1e-14, atol=0)
+
+
+@pytest.mark.parametrize("nx,f", [(8, 0.9), (13, 0.995), (30, 0.95)])
+def test_adjoint_solve_keeps_the_iterate_before_the_stop(nx, f):
+    # after `it` iterations with p.Ap > 0 the solve stops; a solve capped there
+    # takes the same iterations, so its results are the same bits
+    g, x1, w = compressed(nx, f)
+    z = np.zeros_like(w)
+    a = g.step_adjoint(H, x1, z, x1, w, z)
+    print(f"{nx} {f}: {a[3]} iterations, relative residual {a[4]:.2e}", flush=True)
+    assert 0 < a[3] < 4000 and a[4] > 1e-10 and all(np.isfinite(q).all() for q in a[:3])
+    b = g.step_adjoint(H, x1, z, x1, w, z, max_iters=a[3])
+    assert b[3] == a[3] and b[4] == a[4]
+    for p, q in zip(a[:3], b[:3]):
+        assert np.array_equal(p, q)
+
+
+def test_adjoint_solve_with_contact_inverts_a_symmetric_operator():
+    # with contact the product's sum p.Ap is formed after the contact term has
+    # been added.  dL/dv_prev = lambda M / h, and H is symmetric, so lambda_1 .
+    # a_2 = lambda_2 . a_1 for the solves of two right-hand sides.  Bound: each
+    # solve's residual 1e-10 times the condition number is below 1e-6 here,
+    # and the contact term's central difference (1e-6 m along p) is symmetric
+    # to about 1e-6 of it.
+    from closim_amd import scenes as S
+    sc = S.floor_patch(mu=0.0)
+    g = A.converged_solver(sc, "fp64")
+    for _ in range(40):
+        g.step(H)
+    x1, z = sc.positions.copy(), np.zeros(sc.positions.size)
+    rng = np.random.default_rng(2)
+    a1, a2 = rng.standard_normal(z.size), rng.standard_normal(z.size)
+    m = np.repeat(sc.mesh.masses.astype(np.float64), 3)
+    r1 = g.step_adjoint(H, x1, z, x1, a1, z)
+    r2 = g.step_adjoint(H, x1, z, x1, a2, z)
+    assert r1[4] <= 1e-10 and r2[4] <= 1e-10
+    l1, l2 = r1[1] * H / m, r2[1] * H / m
+    p, q = float(l1 @ a2), float(l2 @ a1)
+    print(f"{r1[3]} and {r2[3]} iterations, {p:.12e} {q:.12e}", flush=True)
+    assert abs(p - q) <= 1e-5 * np.sqrt(float(l1 @ a1) * float(l2 @ a2))
+    # the contact is felt: without it lambda differs
+    f2 = S.floor_patch(mu=0.0)
+    f2.contact = None
+    f = A.converged_solver(f2, "fp64")
+    l0 = f.step_adjoint(H, x1, z, x1, a1, z)[1] * H / m
+    assert np.linalg.norm(l0 - l1) > 1e-2 * np.linalg.norm(l1)
