@@ -191,3 +191,23 @@ def test_rule_looks_at_the_vertex_with_the_most_contacts(fine, one_launch):
     g.probe_exchange_wait(0)  # the one-launch solve, where it is tried, gives up at once
     g.step(H)
     assert g.probe_exchange_wait(0xFFFFFFFF) == one_launch
+
+
+@pytest.mark.parametrize("fine,groups", [(5, False), (6, True), (9, True)])
+def test_contact_sums_on_both_sides_of_their_rule(fine, groups):
+    # 15 and 25 entries a vertex on average, 1,100 to 4,800 on one: the sums by a
+    # thread per component and by a work-group (in several rounds of 256)
+    kw = dict(newton_iters=2)
+    sc = grid_below(12, fine)
+    g = HipSolver("fp64", **kw)
+    g.initialize(sc)
+    ids, _, _ = g.probe_active_set(sc.positions, sc.positions)
+    v = np.concatenate([ids[ids[:, 0] == 0][:, 1:5].ravel(), ids[ids[:, 0] == 1][:, 2:6].ravel(),
+                        ids[ids[:, 0] == 2][:, 1]])
+    n = np.bincount(v[v >= 0])
+    print(f"{n.sum()} entries, {(n > 0).sum()} vertices, {n.max()} on one", flush=True)
+    assert (n.sum() >= 16 * (n > 0).sum()) == groups and n.max() > 512
+    g.step(H)
+    o = O.OracleSolver(grid_below(12, fine), _abi.options(**kw))
+    o.step(H)
+    assert np.array_equal(g.getPositions(), o.getPositions()) and np.array_equal(g.getVelocities(), o.getVelocities())
