@@ -64,7 +64,13 @@ enum { CS_PRECOND_JACOBI = 0, CS_PRECOND_BLOCK_JACOBI = 1, CS_PRECOND_SCHWARZ = 
  * CS_PRECOND_SCHWARZ. */
 enum { CS_COARSE_NONE = 0, CS_COARSE_JACOBI = 1, CS_COARSE_BLOCK = 2, CS_COARSE_PCG = 3 };
 
-#define CS_FLAG_TIMING 1u   /* record per-kernel HIP event timings (cs_kernel_timing) */
+/* Record per-kernel HIP event timings (cs_kernel_timing).  The events bracket
+ * the launches of the separate kernels, so the inner solves run as those
+ * kernels also where a step without the flag solves in one launch (FP64
+ * meshes of up to 4,096 vertices and mixed ones of up to 64 HVP tiles, see
+ * CS_FLAG_EAGER): there the times are not those of the untimed step.  The
+ * results are the same. */
+#define CS_FLAG_TIMING 1u
 /* Root polish (not in the reference): when every Armijo trial of a Newton
  * iteration fails, take a full Newton step of the complete Hessian instead
  * (analytic membrane, central differences of bending and contact) if it passes
@@ -74,9 +80,12 @@ enum { CS_COARSE_NONE = 0, CS_COARSE_JACOBI = 1, CS_COARSE_BLOCK = 2, CS_COARSE_
  * differentiated with cs_step_adjoint need the root to grad_tol. */
 #define CS_FLAG_POLISH_ROOT 2u
 /* Launch the mixed-precision PCG iterations one kernel at a time.  By default
- * they run as a captured HIP graph of 8 iterations replayed until the solve
- * converges (same kernels, same order, same results); CS_FLAG_TIMING also
- * selects the one-by-one launches. */
+ * a solve of up to 64 HVP tiles without contact and Schwarz is one launch, and
+ * the others run as a captured HIP graph of 8 iterations (the same kernels in
+ * the same order) replayed until the solve converges; the results are the same
+ * either way.  CS_FLAG_TIMING also selects the one-by-one launches.  (FP64
+ * solves of up to 4,096 vertices, with few contacts a vertex and without
+ * Schwarz, are one launch unless CS_FLAG_TIMING is set.) */
 #define CS_FLAG_EAGER 4u
 /* Newton direction with the analytic membrane Hessian whose stress term is
  * projected to positive semidefinite per triangle (tension only; not in the
@@ -97,8 +106,9 @@ enum { CS_COARSE_NONE = 0, CS_COARSE_JACOBI = 1, CS_COARSE_BLOCK = 2, CS_COARSE_
  * batches of 1, 2, 4, 8 (the reference's batched candidates, shaders/
  * armijo.wgsl:48-238) with one host read per batch; the same results.  Off
  * by default: a trial costs a whole contact check, so the trials computed
- * past the accepted one cost more than the host reads they save (the
- * 512x512 fold runs 13.0 steps/s without, 11.6 with). */
+ * past the accepted one cost more than the host reads they save (ms a step
+ * without and with it: 512x512 fold 40.8 and 43.6 mixed, 60.2 and 61.9 FP64;
+ * 256x256 drape 19.9 and 20.4 mixed, 23.1 and 23.6 FP64). */
 #define CS_FLAG_ARMIJO_SPECULATE 128u
 /* The descent gate of the reference's WebGPU Newton (src/backend/webgpu/
  * gpu-solver.ts:1168-1188, shaders/newton-control.wgsl:58-73) instead of
